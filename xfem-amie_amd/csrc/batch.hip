@@ -93,6 +93,7 @@ size_t Batch::bytes() const
                            &row_cptr, &row_contrib, &persist};
     size_t s = 0;
     for (auto b : all) s += b->n;
+    for (auto &t : team_plans) s += t->bytes();
     return s;
 }
 
@@ -172,11 +173,13 @@ int Batch::grid(int64_t tiles) const
 // on the batch stream; the host lists stay valid until the next call).
 int Batch::set_active(const std::vector<char> &probs)
 {
+    std::vector<int32_t> list;
+    for (int p = 0; p < nprob; p++)
+        if (probs[p]) list.push_back(p);
+    if (!list.empty() && list == h_active_prob) return AMIE_OK;   // as they are on the device
     h_active.clear();
-    h_active_prob.clear();
-    for (int p = 0; p < nprob; p++) {
-        if (!probs[p]) continue;
-        h_active_prob.push_back(p);
+    h_active_prob.swap(list);
+    for (int p : h_active_prob) {
         for (int t = 0; t < ph[p].ntiles; t++) h_active.push_back(ph[p].tile0 + t);
     }
     h_nactive_pinned[0] = (int32_t)h_active.size();
@@ -270,7 +273,7 @@ static int alloc_vectors(Batch &B)
     AMIE_HIP(hipHostMalloc((void **)&B.h_prob_pinned, B.nprob * sizeof(ProbDev), hipHostMallocDefault));
     AMIE_HIP(hipHostMalloc((void **)&B.h_nactive_pinned, 2 * sizeof(int32_t), hipHostMallocDefault));
     if (!B.persist.alloc(16)) return AMIE_ERR_NOMEM;
-    AMIE_HIP(hipHostMalloc((void **)&B.h_persist_pinned, 2 * sizeof(int32_t), hipHostMallocDefault));
+    AMIE_HIP(hipHostMalloc((void **)&B.h_persist_pinned, 4 * sizeof(int32_t), hipHostMallocDefault));
     B.h_prob.resize(B.nprob);
     for (int p = 0; p < B.nprob; p++) {
         ProbDev &P = B.h_prob[p];
@@ -305,18 +308,18 @@ static int build_sell(Batch &B, std::vector<Tmp> &tmp)
         slices += P.nslices;
         tiles += P.ntiles;
     }
-    if (slots >= (int64_t)UINT32_MAX || slices * WAVE >= (int64_t)INT32_MAX) {
+    if (slots + WAVE >= (int64_t)UINT32_MAX || slices * WAVE >= (int64_t)INT32_MAX) {
         set_error("batch too large for 32-bit slot / row indices");
         return AMIE_ERR_ARG;
     }
     B.nslices = slices;
     B.ntiles = tiles;
-    B.nslots = slots;
+    B.nslots = slots + WAVE;   // the last 64 belong to no slice: zero blocks, the null slots of the team CG
     B.nrows_pad = slices * WAVE;
     std::vector<int64_t> h_slice_ptr(slices + 1);
     std::vector<int32_t> h_width(slices), h_rows(slices), h_ts0(tiles), h_tns(tiles), h_tprob(tiles);
-    std::vector<uint32_t> h_col(slots);
-    std::vector<int32_t> h_off(slots / WAVE, 0);
+    std::vector<uint32_t> h_col(B.nslots, 0);
+    std::vector<int32_t> h_off(B.nslots / WAVE, 0);
     std::vector<int64_t> h_dslot(B.nrows_pad);
     std::vector<int32_t> h_rowlen(B.nrows_pad, 0);
 #pragma omp parallel for schedule(dynamic, 1)
@@ -393,6 +396,7 @@ static int build_sell(Batch &B, std::vector<Tmp> &tmp)
         }
     }
     h_slice_ptr[slices] = slots;
+    for (int32_t w : h_width) B.max_width = std::max(B.max_width, w);
     int rc;
     if ((rc = alloc_and_upload(B.slice_ptr, h_slice_ptr.data(), h_slice_ptr.size() * 8))) return rc;
     if ((rc = alloc_and_upload(B.slice_width, h_width.data(), h_width.size() * 4))) return rc;
@@ -714,9 +718,12 @@ template <int Bk> static void launch_post(Batch &B)
 int Batch::ensure_pre64(int mode)
 {
     if ((mode != AMIE_FP64 && mode != AMIE_MIXED_K64) || pre64_ok) return AMIE_OK;
-    if (!vs64.n && !vs64.alloc(nslots * slot_bytes(true, et.b))) {
-        set_error("out of device memory for the scaled FP64 matrix");
-        return AMIE_ERR_NOMEM;
+    if (!vs64.n) {
+        if (!vs64.alloc(nslots * slot_bytes(true, et.b))) {
+            set_error("out of device memory for the scaled FP64 matrix");
+            return AMIE_ERR_NOMEM;
+        }
+        AMIE_HIP(hipMemsetAsync(vs64.p, 0, vs64.n, stream));   // the null slots stay zero
     }
     SolveArgs a = args(AMIE_FP64);
     auto go = [&](auto kern) {
@@ -1058,19 +1065,18 @@ int Batch::start_pass(int mode, const std::vector<char> &subset)
         }
     }
     AMIE_HIP(hipMemcpyAsync(prob.p, h_prob.data(), nprob * sizeof(ProbDev), hipMemcpyHostToDevice, s));
-    AMIE_HIP(hipMemsetAsync(y.p, 0, y.n, s));
-    AMIE_HIP(hipMemsetAsync(p.p, 0, p.n, s));
-    AMIE_HIP(hipMemsetAsync(p2.p, 0, p2.n, s));
-    AMIE_HIP(hipMemsetAsync(p3.p, 0, p3.n, s));
-    AMIE_HIP(hipMemsetAsync(p4.p, 0, p4.n, s));
-    int rc = set_active(subset);
-    if (rc) return rc;
-    R.gt = (int)h_active.size();
-    R.gp = (int)h_active_prob.size();
-    launch0(R.K.norms, R.gt, s, R.a);
-    launch0(R.K.norms_final, R.gp, s, R.a);
-    launch0(R.K.cx, R.gt, s, R.a);
-    launch0(R.K.cr, R.gt, s, R.a);
+    if (int rc = team_prepare(*this, R, subset)) return rc;
+    if (!R.team) {
+        team_dirty = true;
+        for (DevBuf *v : {&y, &p, &p2, &p3, &p4}) AMIE_HIP(hipMemsetAsync(v->p, 0, v->n, s));
+        if (int rc = set_active(subset)) return rc;
+        R.gt = (int)h_active.size();
+        R.gp = (int)h_active_prob.size();
+        launch0(R.K.norms, R.gt, s, R.a);
+        launch0(R.K.norms_final, R.gp, s, R.a);
+        launch0(R.K.cx, R.gt, s, R.a);
+        launch0(R.K.cr, R.gt, s, R.a);
+    }
     R.exec = nullptr;
     R.pgrid = 0;
     R.persist_launched = false;
@@ -1123,9 +1129,13 @@ int Batch::solve_advance()
     if (!R.started || R.finished || R.in_flight) return AMIE_OK;
     hipStream_t s = stream;
     R.nt = 0;
-    if (R.pgrid) {
+    if (R.pgrid || R.team) {
         // the whole pass in one launch; the status copy follows it
-        if (!R.persist_launched) {
+        if (!R.persist_launched && R.team) {
+            if (int rc = team_launch(*this, R)) return rc;
+            R.persist_launched = true;
+            R.periods = R.max_periods;
+        } else if (!R.persist_launched) {
             AMIE_HIP(hipMemsetAsync(persist.p, 0, persist.n, s));
             PersistArgs pa;
             pa.bar = persist.as<unsigned long long>();
@@ -1135,7 +1145,7 @@ int Batch::solve_advance()
             pa.max_periods = (int)std::min<int64_t>(INT32_MAX, std::max<int64_t>(0, R.max_periods - R.periods));
             void *kargs[] = {&R.a, &pa};
             AMIE_HIP(hipLaunchCooperativeKernel((const void *)R.K.kp, dim3(R.pgrid), dim3(WG), kargs, 0, s));
-            AMIE_HIP(hipMemcpyAsync(h_persist_pinned, persist.as<char>() + 8, 8, hipMemcpyDeviceToHost, s));
+            AMIE_HIP(hipMemcpyAsync(h_persist_pinned, persist.p, 16, hipMemcpyDeviceToHost, s));
             R.persist_launched = true;
             R.periods = R.max_periods;
         }
@@ -1168,10 +1178,12 @@ int Batch::solve_poll(bool wait, bool *finished)
         if (!hip_ok(q, "hipEventQuery")) return AMIE_ERR_HIP;
     }
     R.in_flight = false;
-    if (R.pgrid && h_persist_pinned[0]) {
-        set_error("persistent solve: a barrier wait gave up (workgroups not all resident?)");
+    if ((R.pgrid || R.team) && h_persist_pinned[2]) {
+        if (R.team) team_seq = UINT32_MAX;   // the words' state is unknown: the next pass clears them
+        set_error("%s: a wait gave up (workgroups not all resident?)", R.team ? "team solve" : "persistent solve");
         return AMIE_ERR_HIP;
     }
+    if (R.team) team_seq = (uint32_t)h_persist_pinned[3];
     for (int i = 0; i < R.nt; i++) {
         float ms = 0.f, ms2 = 0.f;
         AMIE_HIP(hipEventElapsedTime(&ms, R.tev[4 * i], R.tev[4 * i + 1]));

@@ -5,6 +5,7 @@
 #include <atomic>
 #include <cstdint>
 #include <map>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -74,6 +75,20 @@ struct K1Choice {
     double us = 0.;          // its time per launch with every tile active
 };
 
+// The cut of a batch's problems into members of the team CG (team.hpp).
+struct TeamPlan {
+    int tpw = 0;                     // tiles per member
+    bool ok = false;                 // the problems fit
+    int64_t lds_units = 0;           // largest member's own rows + 2 x halo rows
+    std::vector<int32_t> first;      // per problem: its first member (one more at the end)
+    std::vector<int32_t> h_order;    // members in the order they are claimed, as on the device
+    DevBuf members, order, mslice, mtile, lidx, halo, exported, xb;
+    size_t bytes() const
+    {
+        return members.n + order.n + mslice.n + mtile.n + lidx.n + halo.n + exported.n + xb.n;
+    }
+};
+
 struct SolveRun {
     amie_solve_opts o{};
     int mode = 0;            // precision of the current pass
@@ -95,7 +110,11 @@ struct SolveRun {
     hipEvent_t e0 = nullptr, e1 = nullptr, ev_status = nullptr;
     bool started = false, in_flight = false, finished = false;
     int pgrid = 0;                   // > 0: this pass runs as one persistent launch of pgrid workgroups
-    bool persist_launched = false;
+    TeamPlan *team = nullptr;        // this pass runs as one launch of the team CG
+    const void *team_fn = nullptr;
+    size_t team_lds = 0;             // its dynamic LDS
+    bool team_single = false;        // every team is one workgroup
+    bool persist_launched = false;   // either launch is queued
     amie_solve_stats stats{};
 };
 
@@ -123,6 +142,7 @@ struct Batch {
     int nrhs = 1;
     int nprob = 0;
     std::vector<ProbHost> ph;
+    int32_t max_width = 0;            // blocks of the widest slice
     int64_t nslices = 0, ntiles = 0, nrows_pad = 0, nslots = 0, nelem = 0, nnodes_geo = 0;
     bool has_elements = false, has_macro = false, has_damage_state = false;
     bool fix48_ok = false;            // the last assembly's scaled values fit the fixed-point range
@@ -172,8 +192,12 @@ struct Batch {
     std::vector<ProbDev> h_prob;
     ProbDev *h_prob_pinned = nullptr;
     int32_t *h_nactive_pinned = nullptr;   // [0] tiles, [1] problems
-    DevBuf persist;                        // persistent solve: barrier count (8 bytes), error flag, periods
-    int32_t *h_persist_pinned = nullptr;   // [0] error flag, [1] periods run
+    DevBuf persist;                        // persistent solve: barrier count (8 bytes), error flag, periods;
+                                           // team CG: ticket, progress, error flag, largest sequence number
+    int32_t *h_persist_pinned = nullptr;   // its copy: [2] error flag, [3] periods run or sequence number
+    std::vector<std::unique_ptr<TeamPlan>> team_plans;
+    uint32_t team_seq = 0;                 // sequence numbers the team CG has used
+    bool team_dirty = true;                // p2, p3, p4, y hold launch-path vectors
 
     // captured iteration chunks, keyed by solve variant
     struct GraphEntry {
@@ -203,6 +227,10 @@ struct Batch {
     int k1_format(int mode, bool bj) const;
     int64_t vplane() const { return nrows_pad * et.b; }
 };
+
+// The team CG: whether a pass runs as one (run.team), and its launch.
+int team_prepare(Batch &B, SolveRun &R, const std::vector<char> &subset);
+int team_launch(Batch &B, SolveRun &R);
 
 // Builds the value-indexed FIX48 matrix of the current assembly (dict_ok
 // tells whether it exists: at most DICT_MAX distinct blocks).

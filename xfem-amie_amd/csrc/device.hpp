@@ -708,6 +708,11 @@ template <typename W> __device__ inline const W *cvw(const void *p) { return rei
 // the plane set of p_k
 __device__ inline void *p_planes(const SolveArgs &a, int64_t k) { return a.pset[k & (YGROUP - 1)]; }
 
+// a b + c in one rounding.  The iteration writes its multiply-adds out: left
+// to contraction, two kernels of the same formula may round differently.
+__device__ inline float mac(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ inline double mac(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 // z = M v with M the row's inverse diagonal block (BJ) or the identity.
 template <typename W, int B, bool BJ> __device__ inline void precond(const W *mi, const W *v, W *z)
 {
@@ -716,7 +721,7 @@ template <typename W, int B, bool BJ> __device__ inline void precond(const W *mi
         if (BJ) {
             W s = 0;
 #pragma unroll
-            for (int j = 0; j < B; j++) s += mi[i * B + j] * v[j];
+            for (int j = 0; j < B; j++) s = mac(mi[i * B + j], v[j], s);
             z[i] = s;
         } else {
             z[i] = v[i];
@@ -779,7 +784,7 @@ __device__ inline void spmv_row(const SolveArgs &a, const void *vals, int s, int
                     for (int i = 0; i < B; i++) {
                         const A m = (A)BR::at(blk[u], j * B + i);
 #pragma unroll
-                        for (int r = 0; r < NR; r++) acc[r][i] += m * xv[r][j];
+                        for (int r = 0; r < NR; r++) acc[r][i] = mac(m, xv[r][j], acc[r][i]);
                     }
             }
     }
@@ -874,7 +879,7 @@ __device__ inline void spmv_slice(const SolveArgs &a, const void *vals, int64_t 
                         if constexpr (IS_DICT) m = (A)dv[j * B + i];
                         else m = (A)BR::at(blk[u], j * B + i);
 #pragma unroll
-                        for (int r = 0; r < NR; r++) acc[r][i] += m * xv[r][j];
+                        for (int r = 0; r < NR; r++) acc[r][i] = mac(m, xv[r][j], acc[r][i]);
                     }
             }
     }
@@ -954,9 +959,9 @@ __device__ inline void spmv_tile(const SolveArgs &a, const void *vals, int t, co
                 precond<W, B, BJ>(mi, qv, mq);
 #pragma unroll
                 for (int i = 0; i < B; i++) {
-                    part[k] += (double)pv[k][i] * (double)qv[i];
-                    part[NR + k] += (double)qv[i] * (double)zv[i];
-                    part[2 * NR + k] += (double)qv[i] * (double)mq[i];
+                    part[k] = mac((double)pv[k][i], (double)qv[i], part[k]);
+                    part[NR + k] = mac((double)qv[i], (double)zv[i], part[NR + k]);
+                    part[2 * NR + k] = mac((double)qv[i], (double)mq[i], part[2 * NR + k]);
                 }
             }
         }
@@ -990,6 +995,88 @@ __global__ __launch_bounds__(WG) void k_spmv(SolveArgs a)
 }
 
 // ------------------------------------------- R: per-problem CG scalars
+// The scalars of right-hand side k (one thread) from the SpMV sums (p.q, q.z,
+// q.Mq) and the residual sums (r.z, r.r, and after a refinement, ck,
+// |b - K x|^2 and |S (b - K x)|^2); returns what it found as R_* bits.
+enum { R_BUSY = 1, R_BAD = 2, R_STALLED = 4, R_NEED = 8, R_LADDER = 16 };
+__device__ inline int reduce_rhs(ProbDev &P, int k, double pq, double qz, double qmq, double rho, double rr,
+                                 double rr64, double rs2, bool ck)
+{
+    if (P.done[k]) {
+        P.alpha[k] = P.beta[k] = 0.;
+        return 0;
+    }
+    int f = 0;
+    if (ck) {
+        // accuracy floor: the true (replaced) rho well above the
+        // recurrence's prediction for the same residual means the working
+        // precision can no longer follow the iteration.  The split matrix
+        // hands over to the FP64 matrix; otherwise the problem is stalled
+        // (and continues in FP64 when escalation is on).
+        if (P.rho_pred[k] > 0. && rho > 4. * P.rho_pred[k]) {
+            if (P.ladder && !P.kmode) f |= R_LADDER;
+            else if (P.stall_iters > 0) f |= R_STALLED;
+        }
+        // the refinement's FP64 residual decides convergence
+        if (!(rr64 == rr64)) f |= R_BAD;
+        const double rel = P.bb64[k] > 0. ? sqrt(rr64 / P.bb64[k]) : sqrt(rr64);
+        P.relres[k] = P.relres_out[k] = rel;
+        P.rr_ckpt[k] = rr;
+        // the stop measure and its bound: relative FP64 residual, or the
+        // reference's absolute sqrt(r . D^-1 r) = ||S r64||
+        const double meas = P.ref_eps > 0. ? sqrt(rs2) : rel;
+        const double bound = P.ref_eps > 0. ? fmax(1e-12, P.ref_eps) : P.rtol;
+        if (meas <= bound) {
+            P.done[k] = P.done_out[k] = 1;
+            P.alpha[k] = P.beta[k] = 0.;
+            return f;
+        }
+        // expected working-precision r.r at convergence, from this ratio
+        P.rr_target[k] = rr * (bound / meas) * (bound / meas);
+        if (rel < 0.5 * P.rel_best[k]) {
+            P.rel_best[k] = rel;
+            P.best_it[k] = P.iters;
+        } else if (P.stall_iters > 0 && P.iters - P.best_it[k] >= P.stall_iters) {
+            f |= R_STALLED;
+        }
+    }
+    f |= R_BUSY;
+    if (!(pq == pq) || !(rho == rho) || !(qz == qz) || !(qmq == qmq)) f |= R_BAD;
+    const double alpha = pq != 0. ? rho / pq : 0.;
+    const double rho1 = mac(alpha * alpha, qmq, mac(-2. * alpha, qz, rho));
+    P.alpha[k] = alpha;
+    P.alpha_ring[k][P.iters & (YGROUP - 1)] = alpha;
+    P.beta[k] = rho != 0. ? rho1 / rho : 0.;
+    P.rho_pred[k] = rho1;
+    P.rr[k] = rr;
+    if (rr < P.drop * P.drop * P.rr_ckpt[k]) f |= R_NEED;   // FP32 residual dropped: refine
+    if (rr <= P.rr_target[k]) f |= R_NEED;                   // may have converged: confirm in FP64
+    return f;
+}
+
+// The problem's decisions (one thread) from its right-hand sides' bits.
+__device__ inline void reduce_finish(ProbDev &P, int f, bool ck)
+{
+    if (f & R_LADDER) P.kmode = 1;
+    if (P.kmode) P.iters_k64 += 1;
+    if (ck) {
+        P.nckpt += 1;
+        P.last_ckpt = P.iters;
+        P.ckpt_pending = 0;
+        P.src_ckpt = 0;
+        P.first = 0;
+    }
+    if (f & R_BAD) { P.status = ST_NAN; return; }
+    if (!(f & R_BUSY)) { P.status = ST_CONVERGED; return; }
+    if (ck && P.iters >= P.maxit) { P.status = ST_MAXIT; return; }
+    if (f & R_STALLED) { P.status = ST_STALLED; return; }
+    // the previous update deferred its y term (one more pending) or added
+    // every pending one; a refinement added everything
+    P.ypend = (ck || P.ypend == YGROUP - 1) ? 0 : P.ypend + 1;
+    P.iters += 1;
+    if ((f & R_NEED) || P.iters >= P.maxit || P.iters - P.last_ckpt >= P.ckpt_interval) P.ckpt_pending = 1;
+}
+
 // One workgroup per active problem.  Consumes the residual partials of the
 // previous update (or refinement) and this iteration's SpMV partials.
 template <int NR>
@@ -1003,79 +1090,11 @@ __device__ inline void reduce_body(const SolveArgs &a, int pi)
     if (ck) problem_sums2<3 * NR, 4 * NR>(a.part1, a.partc, P, s1, s0, lds2);
     else problem_sums2<3 * NR, 2 * NR>(a.part1, a.part2, P, s1, s0, lds2);
     if (threadIdx.x != 0) return;
-    bool all = true, bad = false, stalled = false, need = false, ladder_up = false;
-    for (int k = 0; k < NR; k++) {
-        if (P.done[k]) {
-            P.alpha[k] = P.beta[k] = 0.;
-            continue;
-        }
-        const double rho = s0[k], rr = s0[NR + k];
-        if (ck) {
-            // accuracy floor: the true (replaced) rho well above the
-            // recurrence's prediction for the same residual means the working
-            // precision can no longer follow the iteration.  The split matrix
-            // hands over to the FP64 matrix; otherwise the problem is stalled
-            // (and continues in FP64 when escalation is on).
-            if (P.rho_pred[k] > 0. && s0[k] > 4. * P.rho_pred[k]) {
-                if (P.ladder && !P.kmode) ladder_up = true;
-                else if (P.stall_iters > 0) stalled = true;
-            }
-            // the refinement's FP64 residual decides convergence
-            const double rr64 = s0[2 * NR + k];
-            if (!(rr64 == rr64)) bad = true;
-            const double rel = P.bb64[k] > 0. ? sqrt(rr64 / P.bb64[k]) : sqrt(rr64);
-            P.relres[k] = P.relres_out[k] = rel;
-            P.rr_ckpt[k] = rr;
-            // the stop measure and its bound: relative FP64 residual, or the
-            // reference's absolute sqrt(r . D^-1 r) = ||S r64||
-            const double meas = P.ref_eps > 0. ? sqrt(s0[3 * NR + k]) : rel;
-            const double bound = P.ref_eps > 0. ? fmax(1e-12, P.ref_eps) : P.rtol;
-            if (meas <= bound) {
-                P.done[k] = P.done_out[k] = 1;
-                P.alpha[k] = P.beta[k] = 0.;
-                continue;
-            }
-            // expected working-precision r.r at convergence, from this ratio
-            P.rr_target[k] = rr * (bound / meas) * (bound / meas);
-            if (rel < 0.5 * P.rel_best[k]) {
-                P.rel_best[k] = rel;
-                P.best_it[k] = P.iters;
-            } else if (P.stall_iters > 0 && P.iters - P.best_it[k] >= P.stall_iters) {
-                stalled = true;
-            }
-        }
-        all = false;
-        const double pq = s1[k], qz = s1[NR + k], qmq = s1[2 * NR + k];
-        if (!(pq == pq) || !(rho == rho) || !(qz == qz) || !(qmq == qmq)) bad = true;
-        const double alpha = pq != 0. ? rho / pq : 0.;
-        const double rho1 = rho - 2. * alpha * qz + alpha * alpha * qmq;
-        P.alpha[k] = alpha;
-        P.alpha_ring[k][P.iters & (YGROUP - 1)] = alpha;
-        P.beta[k] = rho != 0. ? rho1 / rho : 0.;
-        P.rho_pred[k] = rho1;
-        P.rr[k] = rr;
-        if (rr < P.drop * P.drop * P.rr_ckpt[k]) need = true;   // FP32 residual dropped: refine
-        if (rr <= P.rr_target[k]) need = true;                   // may have converged: confirm in FP64
-    }
-    if (ladder_up) P.kmode = 1;
-    if (P.kmode) P.iters_k64 += 1;
-    if (ck) {
-        P.nckpt += 1;
-        P.last_ckpt = P.iters;
-        P.ckpt_pending = 0;
-        P.src_ckpt = 0;
-        P.first = 0;
-    }
-    if (bad) { P.status = ST_NAN; return; }
-    if (all) { P.status = ST_CONVERGED; return; }
-    if (ck && P.iters >= P.maxit) { P.status = ST_MAXIT; return; }
-    if (stalled) { P.status = ST_STALLED; return; }
-    // the previous update deferred its y term (one more pending) or added
-    // every pending one; a refinement added everything
-    P.ypend = (ck || P.ypend == YGROUP - 1) ? 0 : P.ypend + 1;
-    P.iters += 1;
-    if (P.iters >= P.maxit || P.iters - P.last_ckpt >= P.ckpt_interval) need = true;
-    if (need) P.ckpt_pending = 1;
+    int f = 0;
+    for (int k = 0; k < NR; k++)
+        f |= reduce_rhs(P, k, s1[k], s1[NR + k], s1[2 * NR + k], s0[k], s0[NR + k], ck ? s0[2 * NR + k] : 0.,
+                        ck ? s0[3 * NR + k] : 0., ck);
+    reduce_finish(P, f, ck);
 }
 
 template <int NR>
@@ -1136,10 +1155,10 @@ __device__ inline void k2_body(const SolveArgs &a, int t, int slot)
                         Node<W, B, true>::load(cvw<W>(p_planes(a, k_it - j)) + idx, pp);
                         const double alp = P.alpha_ring[k][(k_it - j) & (YGROUP - 1)];
 #pragma unroll
-                        for (int i = 0; i < B; i++) yv[i] += alp * (double)pp[i];
+                        for (int i = 0; i < B; i++) yv[i] = mac(alp, (double)pp[i], yv[i]);
                     }
 #pragma unroll
-                    for (int i = 0; i < B; i++) yv[i] += al64 * (double)pv[i];
+                    for (int i = 0; i < B; i++) yv[i] = mac(al64, (double)pv[i], yv[i]);
                     Node<double, B, true>::store(y + idx, yv);
                 }
                 if (ck) continue;
@@ -1147,14 +1166,14 @@ __device__ inline void k2_body(const SolveArgs &a, int t, int slot)
                 Node<W, B, true>::load(q + idx, qv);
                 Node<W, B, true>::load(r + idx, rv);
 #pragma unroll
-                for (int i = 0; i < B; i++) rv[i] -= al * qv[i];
+                for (int i = 0; i < B; i++) rv[i] = mac(-al, qv[i], rv[i]);
                 Node<W, B, true>::store(r + idx, rv);
                 precond<W, B, BJ>(mi, rv, zv);
 #pragma unroll
                 for (int i = 0; i < B; i++) {
-                    pv[i] = zv[i] + be * pv[i];
-                    part[k] += (double)rv[i] * (double)zv[i];
-                    part[NR + k] += (double)rv[i] * (double)rv[i];
+                    pv[i] = mac(be, pv[i], zv[i]);
+                    part[k] = mac((double)rv[i], (double)zv[i], part[k]);
+                    part[NR + k] = mac((double)rv[i], (double)rv[i], part[NR + k]);
                 }
                 Node<W, B, true>::store(pn + idx, pv);
             }
@@ -1195,7 +1214,7 @@ __device__ inline void cx_body(const SolveArgs &a, int t)
         Node<double, B>::load(a.x64 + idx, xv);
 #pragma unroll
         for (int i = 0; i < B; i++) {
-            xv[i] += sr[i] * yv[i];
+            xv[i] = mac(sr[i], yv[i], xv[i]);
             yv[i] = 0;
         }
         Node<double, B>::store(a.x64 + idx, xv);
@@ -1258,8 +1277,8 @@ __device__ inline void cr_body(const SolveArgs &a, int t)
                 for (int i = 0; i < B; i++) {
                     const double r64 = bv[i] - acc[k][i];
                     const double rs = sr[i] * r64;
-                    part[2 * NR + k] += r64 * r64;
-                    part[3 * NR + k] += rs * rs;
+                    part[2 * NR + k] = mac(r64, r64, part[2 * NR + k]);
+                    part[3 * NR + k] = mac(rs, rs, part[3 * NR + k]);
                     rv[i] = (W)rs;
                 }
                 Node<W, B>::store(r + idx, rv);
@@ -1267,9 +1286,9 @@ __device__ inline void cr_body(const SolveArgs &a, int t)
                 Node<W, B>::load(pk + idx, pv);
 #pragma unroll
                 for (int i = 0; i < B; i++) {
-                    pv[i] = zv[i] + be * pv[i];
-                    part[k] += (double)rv[i] * (double)zv[i];
-                    part[NR + k] += (double)rv[i] * (double)rv[i];
+                    pv[i] = mac(be, pv[i], zv[i]);
+                    part[k] = mac((double)rv[i], (double)zv[i], part[k]);
+                    part[NR + k] = mac((double)rv[i], (double)rv[i], part[NR + k]);
                 }
                 Node<W, B>::store(pn + idx, pv);
             }
@@ -1660,12 +1679,28 @@ __global__ __launch_bounds__(WG) void k_rhs_norms(SolveArgs a)
                 for (int i = 0; i < B; i++) {
                     const double bv = a.b64[k * a.vplane + (size_t)row * B + i];
                     const double sb = a.S[(size_t)row * B + i] * bv;
-                    part[k] += sb * sb;
-                    part[NR + k] += bv * bv;
+                    part[k] = mac(sb, sb, part[k]);
+                    part[NR + k] = mac(bv, bv, part[NR + k]);
                 }
         }
     }
     write_partials<2 * NR>(part, a.partn, t, lds);
+}
+
+// The stopping measures of one problem (one thread) from |S b|^2 and |b|^2.
+template <int NR> __device__ inline void norm_scalars(ProbDev &P, const double *sums)
+{
+    for (int k = 0; k < NR; k++) {
+        P.bb[k] = sums[k];
+        P.bb64[k] = sums[NR + k];
+        P.rr_target[k] = P.ref_eps > 0. ? fmax(1e-24, P.ref_eps * P.ref_eps) : P.rtol * P.rtol * sums[k];
+        // a homogeneous right-hand side is solved by x = 0
+        // (solvers/conjugategradient.cpp:74-78)
+        if (sums[NR + k] == 0.) {
+            P.done[k] = P.done_out[k] = 1;
+            P.relres[k] = P.relres_out[k] = 0.;
+        }
+    }
 }
 
 // One workgroup per active problem: |S b|^2 and |b|^2 from the norm partials.
@@ -1678,18 +1713,7 @@ __global__ __launch_bounds__(WG) void k_norms_final(SolveArgs a)
     if (P.status != ST_RUNNING) return;
     double sums[2 * NR];
     problem_sums<2 * NR>(a.partn, P, sums, lds);
-    if (threadIdx.x != 0) return;
-    for (int k = 0; k < NR; k++) {
-        P.bb[k] = sums[k];
-        P.bb64[k] = sums[NR + k];
-        P.rr_target[k] = P.ref_eps > 0. ? fmax(1e-24, P.ref_eps * P.ref_eps) : P.rtol * P.rtol * sums[k];
-        // a homogeneous right-hand side is solved by x = 0
-        // (solvers/conjugategradient.cpp:74-78)
-        if (sums[NR + k] == 0.) {
-            P.done[k] = P.done_out[k] = 1;
-            P.relres[k] = P.relres_out[k] = 0.;
-        }
-    }
+    if (threadIdx.x == 0) norm_scalars<NR>(P, sums);
 }
 
 // ------------------------------------------------- plain SpMV (test hook)
