@@ -105,7 +105,7 @@ int team_tiles(const Batch &B, int jmax, double slot_bytes)
     int tpw = std::max(1, std::min(4, (int)(160e3 / tile_bytes)));
     int big = 0;
     for (const ProbHost &P : B.ph) big = std::max(big, P.ntiles);
-    if (big <= 4) tpw = std::max(tpw, big);
+    tpw = big <= 4 ? big : tpw;
     tpw = std::min(tpw, most);
     auto members = [&](int t) {
         int64_t n = 0;

@@ -35,13 +35,14 @@
 // exchanges r of the halo rows.
 //
 // Measured on an MI355X, microseconds an iteration, launch path -> team: P1
-// 16^2 FP64 18.2 -> 3.8, P1 128^2 FP64 16.5 -> 5.2, P2 45^2 FIX48 20 -> 8.0, Tet4
-// 19^3 block Jacobi 21 -> 9.6, 64 RVEs of 32..256 cells with three loads
-// 100 -> 49 (value-indexed) and 110 -> 72 (planes), Tet4 64^3 62 -> 49, P2 400^2
-// 61 -> 44.  What bounds it: on small problems the dependent chain of one
-// iteration (SpMV, transposing sums, one exchange, scalars, update); on large
-// ones the latency of the matrix stream at 8 wavefronts a CU, and the spread
-// of the members' times, which the exchange waits for.
+// 16^2 FP64 18.2 -> 2.4, P1 128^2 FP64 16.5 -> 4.5, P2 45^2 FIX48 20 -> 6.7, Tet4
+// 19^3 block Jacobi 21 -> 8.2, P2 250^2 40 -> 13.4, 64 RVEs of 32..256 cells
+// with three loads 100 -> 48 (value-indexed) and 110 -> 71 (planes), Tet4 64^3
+// 62 -> 48, P2 400^2 61 -> 42.  What bounds it: on small problems the dependent
+// chain of one iteration (product, transposing sums, one exchange of 1.5 us,
+// scalars, update); on large ones the latency of the matrix stream at 8
+// wavefronts a CU, and the spread of the members' times, which the exchange
+// waits for.
 //
 // The workgroups of a launch (at most one per CU, launched cooperatively, so
 // all are resident) claim members in a fixed order from a counter, all
@@ -104,12 +105,10 @@ template <> struct TeamWord<float> {
     {
         team_store(l + i, __float_as_uint(v), seq);
     }
-    __device__ static inline bool load(const uint64_t *l, const uint64_t *, size_t i, uint32_t seq, float &v)
-    {
-        const uint64_t a = team_load(l + i);
-        v = __uint_as_float((uint32_t)a);
-        return team_is(a, seq);
-    }
+    uint64_t a;
+    __device__ inline void load(const uint64_t *l, const uint64_t *, size_t i) { a = team_load(l + i); }
+    __device__ inline bool is(uint32_t seq) const { return team_is(a, seq); }
+    __device__ inline float value() const { return __uint_as_float((uint32_t)a); }
 };
 template <> struct TeamWord<double> {
     __device__ static inline void store(uint64_t *l, uint64_t *h, size_t i, double v, uint32_t seq)
@@ -117,12 +116,14 @@ template <> struct TeamWord<double> {
         team_store(l + i, (uint32_t)__double2loint(v), seq);
         team_store(h + i, (uint32_t)__double2hiint(v), seq);
     }
-    __device__ static inline bool load(const uint64_t *l, const uint64_t *h, size_t i, uint32_t seq, double &v)
+    uint64_t a, b;
+    __device__ inline void load(const uint64_t *l, const uint64_t *h, size_t i)
     {
-        const uint64_t a = team_load(l + i), b = team_load(h + i);
-        v = __hiloint2double((int)(uint32_t)b, (int)(uint32_t)a);
-        return team_is(a, seq) && team_is(b, seq);
+        a = team_load(l + i);
+        b = team_load(h + i);
     }
+    __device__ inline bool is(uint32_t seq) const { return team_is(a, seq) && team_is(b, seq); }
+    __device__ inline double value() const { return __hiloint2double((int)(uint32_t)b, (int)(uint32_t)a); }
 };
 
 // One wait: polls counted, and every few thousand the clock.  It gives up
@@ -248,6 +249,7 @@ template <int B> struct TeamBlk<Pre64, B> {
         }
         return k % 2 ? p[k / 2].y : p[k / 2].x;
     }
+    __device__ inline void keep() {}
 };
 template <int B> struct TeamBlk<Fix48, B> {
     typename BlkRaw<Fix48, B>::Raw r;
@@ -267,6 +269,11 @@ template <int B> struct TeamBlk<Fix48, B> {
         }
     }
     __device__ inline double at(const double *, int k) const { return BlkRaw<Fix48, B>::at(r, k); }
+    __device__ inline void keep()
+    {
+        if constexpr (B == 2) asm volatile("" : "+v"(r.l), "+v"(r.h));
+        else asm volatile("" : "+v"(r.l0), "+v"(r.l1), "+v"(r.l2), "+v"(r.h0), "+v"(r.h1));
+    }
 };
 template <int B> struct TeamBlk<Dict, B> {
     uint32_t id;
@@ -275,12 +282,11 @@ template <int B> struct TeamBlk<Dict, B> {
         id = (reinterpret_cast<const uint16_t *>(base) + s0)[lane];
     }
     __device__ inline double at(const double *tab, int k) const { return tab[id * DictEntry<B>::N + k]; }
+    __device__ inline void keep() { asm volatile("" : "+v"(id)); }
 };
 
-// A group of N blocks of a row: 16-37 registers, twice (the next group is
-// loaded while one is multiplied).
-template <typename M, int B, int NR> struct TeamGroup {
-    static constexpr int N = std::is_same<M, Dict>::value ? 8 : (B * NR == 2 ? 4 : 2);
+// A group of N blocks of a row.
+template <typename M, int B, int N> struct TeamGroup {
     uint32_t li[N];
     TeamBlk<M, B> blk[N];
     // blocks from slot s0 on, `left` of them in the row: past it the null
@@ -295,6 +301,48 @@ template <typename M, int B, int NR> struct TeamGroup {
 #pragma unroll
         for (int u = 0; u < N; u++) blk[u].load(vals, ns, s[u], lane);
     }
+};
+
+// The first blocks of a thread's rows stay in registers for the whole solve
+// and the rest of a longer row is streamed: as many blocks, in quads, as the
+// registers beside the rows' state take without spilling.  (Products of 7
+// blocks a row: 2600 -> 1700 cycles of an iteration.  3 x 3 blocks are too
+// large, more than two slices a wavefront too many; of the value-indexed
+// matrix a block is one register.)
+template <typename M, int B, int NR, int J> constexpr int team_resident()
+{
+    if (std::is_same<M, Dict>::value) return J * NR * B <= 8 ? 8 : 0;
+    if (B == 3 || J > 2) return 0;
+    if (NR == 3) return J == 1 ? 8 : 0;
+    return J == 2 ? 8 : (std::is_same<M, Fix48>::value ? 16 : 12);
+}
+template <typename M, int B, int R> struct TeamRes {
+    uint32_t li[R / 2];   // two local columns a register
+    TeamBlk<M, B> blk[R];
+    __device__ inline void load(const uint16_t *lidx, const void *vals, int64_t ns, int64_t s0, int width, int lane)
+    {
+#pragma unroll
+        for (int u = 0; u < R; u++) {
+            const int64_t s = u < width ? s0 + u * WAVE : ns - WAVE;
+            const uint32_t l = (lidx + s)[lane];
+            li[u / 2] = u % 2 ? li[u / 2] | l << 16 : l;
+            blk[u].load(vals, ns, s, lane);
+        }
+    }
+    // Said to change each iteration: addresses and values made from them are
+    // then made again, not kept beside them in registers that spill.
+    __device__ inline void keep(int u0)
+    {
+#pragma unroll
+        for (int u = u0; u < u0 + 4; u++) {
+            if (u % 2 == 0) asm volatile("" : "+v"(li[u / 2]));
+            blk[u].keep();
+        }
+    }
+    __device__ inline uint32_t col(int u) const { return u % 2 ? li[u / 2] >> 16 : li[u / 2] & 0xffffu; }
+};
+template <typename M, int B> struct TeamRes<M, B, 0> {
+    __device__ inline void load(const uint16_t *, const void *, int64_t, int64_t, int, int) {}
 };
 
 // A row's NR x B values (p in LDS, the exchanged words): one record per row,
@@ -360,7 +408,7 @@ struct TeamAll {
     SolveArgs a;
     TeamArgs t;
 };
-// (With one slice a wavefront there is room, and the loads would be latency.)
+// (KEEP: with one slice a wavefront and no resident blocks there is room.)
 typedef const __attribute__((address_space(4))) TeamAll *TeamPtr;
 template <bool KEEP> __device__ inline TeamPtr team_args_of()
 {
@@ -368,6 +416,14 @@ template <bool KEEP> __device__ inline TeamPtr team_args_of()
     if (!KEEP) asm volatile("" : "+s"(p));
     return p;
 }
+
+// lane k's value in every lane
+__device__ inline double lane_value(double v, int k)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), k), __builtin_amdgcn_readlane(__double2loint(v), k));
+}
+
+__device__ inline double lane_at(double v, int k) { return lane_value(v, __builtin_amdgcn_readfirstlane(k)); }
 
 // J: slices per wavefront (wavefront w has the local slices w, w + 8, ...).
 // Registers: y, r, q of J rows, NR B (8 + 2 sizeof(W)) bytes each.
@@ -381,18 +437,30 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
     constexpr int MAXT = TEAM_WAVES * J / TILE_SLICES;   // tiles of a member
     constexpr int MAXV = (NVC + TEAM_WAVES - 1) / TEAM_WAVES;   // values per wavefront
     constexpr int NGRP = TEAM_COLS / WAVE;
+    constexpr int NDIR = NR == 1 ? NGRP : 1;   // groups of 64 tiles summed in one step
     constexpr int REC = NR * B;
     static_assert(MAXT <= 16 && NVC * 16 <= TEAM_WG, "one thread per tile and value");
     extern __shared__ __align__(16) char dyn[];
     __shared__ ProbDev P;
     __shared__ int4 sdesc[TEAM_WAVES * J];                // slot pointer lo, hi, width | rows << 16, slice
-    __shared__ double wsum[TEAM_WAVES * J][NVC];          // sums of a slice
+    __shared__ double wsum[TEAM_WAVES * J][3 * NR];       // sums of a slice: K1's,
+    __shared__ double wres[2][TEAM_WAVES * J][NVC - 3 * NR];   // the residual's (two buffers)
     __shared__ double grp[TEAM_WAVES / NGRP][NGRP];       // sums of 64 columns
-    __shared__ double red[NVC];                           // sums of the problem
+    __shared__ double red_[TEAM_WAVES][NVC];              // sums of the problem (a team of one: per wavefront)
     __shared__ int s_item, s_bad;
     (void)all_;
-    constexpr auto team_args = team_args_of<J == 1>;
-    const int wave = wave_id(), lane = threadIdx.x % WAVE, tid = threadIdx.x;
+    constexpr bool KEEP = J == 1 && team_resident<M, B, NR, J>() == 0;
+    constexpr auto team_args = team_args_of<KEEP>;
+    const int wave = wave_id();
+    int lane = threadIdx.x % WAVE, tid = threadIdx.x;
+    // Said to change, so that lane masks made from them are made where they
+    // are used: kept over the iteration they fill the scalar registers, and
+    // what spills there is read back a lane at a time.
+    // (Measured: 3 % of P1 128^2, the other way by as much where a row has
+    // more values and the scalar work hides.)
+    auto fresh = [&] {
+        if (B == 2 && NR == 1) asm volatile("" : "+v"(lane), "+v"(tid));
+    };
     size_t tab_bytes = 0;
     if constexpr (std::is_same<M, Dict>::value) {
         TeamPtr A = team_args();
@@ -419,14 +487,14 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
             reinterpret_cast<uint32_t *>(&P)[i] = reinterpret_cast<const uint32_t *>(gP)[i];
         const int G = mb.G, rows = mb.nsl * WAVE, H = mb.nhalo;
         const int mytiles = mb.nsl / TILE_SLICES;
-        const bool hop = mb.ntiles > WAVE;     // the sums take two steps (collect)
+        const bool hop = mb.ntiles > NDIR * WAVE;   // the sums take two steps (collect)
         W *lr = lp + REC * (rows + H);         // r of the halo
         uint32_t xs = A0->t.seq0, qs = xs;     // sequence numbers of the sums and of the rows
         uint64_t *const xbase = A0->t.xb + 2 * mb.xb;
         auto xb_at = [&](uint32_t seq, int v, int t) { return xbase + 2 * (((seq & 1) * NVC + v) * mb.ntiles + t); };
         auto total_at = [&](uint32_t seq, int v) { return xbase + 2 * (2 * NVC * mb.ntiles + (seq & 1) * NVC + v); };
         // this thread's tile and value of a publication, and its first halo row
-        const int pt = tid & 15, pv = tid >> 4;
+        const int pt = tid & 15, pv = (NR == 1 ? TEAM_WG - 1 - tid : tid) >> 4;
         const int ptile = pt < mytiles ? A0->t.mtile[mb.mt0 + pt] : 0;
         const int halo_row = tid < H ? (int)A0->t.halo[mb.halo0 + tid] : 0;
         if (tid < TEAM_WAVES * J) {
@@ -473,24 +541,33 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
         W hv[NR][B];   // the thread's first halo row, as collected
 
         // Sums of N values of the wavefront's slice j into wsum, from value vfirst on.
+        // (The residual's: r.z is still read by slow wavefronts of a team of one
+        // when the next update writes it.)
+        int rp = 0;
         auto slice_sums = [&](double *v, auto n, int vfirst, int j) {
             constexpr int N = decltype(n)::value;
             int id;
             const double s = wave_sums<N>(v, lane, id);
-            if ((lane & 1) == 0) wsum[wave + j * TEAM_WAVES][vfirst + id] = s;
+            double *to = vfirst < 3 * NR ? &wsum[wave + j * TEAM_WAVES][vfirst]
+                                         : &wres[rp][wave + j * TEAM_WAVES][vfirst - 3 * NR];
+            if ((lane & 1) == 0) to[id] = s;
         };
         auto tile_sum = [&](int t, int v) {
-            const double *l = &wsum[t * TILE_SLICES][v];
-            return (l[0] + l[NVC]) + (l[2 * NVC] + l[3 * NVC]);
+            const bool k1 = v < 3 * NR;
+            const int ld = k1 ? 3 * NR : NVC - 3 * NR;
+            const double *l = k1 ? &wsum[t * TILE_SLICES][v] : &wres[rp][t * TILE_SLICES][v - 3 * NR];
+            return (l[0] + l[ld]) + (l[2 * ld] + l[3 * ld]);
         };
+        double *const red = red_[G == 1 ? wave : 0];
         auto put_sum = [&](uint64_t *o, double s, uint32_t seq) {
             team_store(o, (uint32_t)__double2loint(s), seq);
             team_store(o + 1, (uint32_t)__double2hiint(s), seq);
         };
         auto poll_sum = [&](const uint64_t *o, uint32_t seq, double &v) {
-            const uint64_t lo = team_load(o), hi = team_load(o + 1);
-            v = __hiloint2double((int)(uint32_t)hi, (int)(uint32_t)lo);
-            return team_is(lo, seq) && team_is(hi, seq);
+            TeamWord<double> w;
+            w.load(o, o + 1, 0);
+            v = w.value();
+            return w.is(seq);
         };
         // Tile sums of values [v0, v1) from wsum, published with number seq
         // (a team of one reads them there).
@@ -498,74 +575,137 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
             const int v = v0 + pv;
             if (G > 1 && pt < mytiles && v < v1) put_sum(xb_at(seq, v, ptile), tile_sum(pt, v), seq);
         };
+        // A row's words.  A poll issues every load before it looks at one (a
+        // wait is for one trip of 900 cycles then, not for one a word), so
+        // lanes with nothing to read read word 0 and ignore it.
+        struct Row {
+            TeamWord<W> w[NR * B];
+            __device__ inline void load(TeamPtr A, uint32_t seq, int gr)
+            {
+                const uint64_t *ql = A->t.ql[seq & 1], *qh = A->t.qh[seq & 1];
+#pragma unroll
+                for (int i = 0; i < NR * B; i++) w[i].load(ql, qh, (size_t)gr * REC + i);
+            }
+            __device__ inline bool get(uint32_t seq, W(*v)[B]) const
+            {
+                bool all = true;
+#pragma unroll
+                for (int i = 0; i < NR * B; i++) {
+                    all &= w[i].is(seq);
+                    v[i / B][i % B] = w[i].value();
+                }
+                return all;
+            }
+        };
         auto poll_row = [&](TeamPtr A, uint32_t seq, int gr, W(*v)[B]) {
-            const uint64_t *ql = A->t.ql[seq & 1], *qh = A->t.qh[seq & 1];
-            bool all = true;
-#pragma unroll
-            for (int k = 0; k < NR; k++)
-#pragma unroll
-                for (int i = 0; i < B; i++)
-                    all &= TeamWord<W>::load(ql, qh, (size_t)gr * REC + k * B + i, seq, v[k][i]);
-            return all;
+            Row w;
+            w.load(A, seq, gr);
+            return w.get(seq, v);
         };
         // The problem's sums of values [0, nv) in problem_sums2's order: columns
         // of the tiles t, t + 256, ... in order, a butterfly over each 64
-        // columns, the four in pairs.  Up to 64 tiles every member reads every
-        // tile's values; beyond (each would read 15 x 16 bytes a tile) value v
-        // is summed by member v % G alone and published once more, a second
-        // step of 1.2 us that 64 members make good.  The sums end in red, for
-        // wavefront 0.  hv receives this thread's first halo row with number
-        // hseq, when that is not 0: its wait is the same one.
+        // columns, the four in pairs.  Up to 256 tiles (64 with three
+        // right-hand sides, whose words would need 100 registers) every member
+        // reads every tile's values; beyond value v is summed by member v % G
+        // alone and published once more, a second step of 1.2 us that 64
+        // members make good.  The sums end in red, for
+        // every wavefront.  hv receives this thread's first halo row with number
+        // hseq, when that is not 0: its wait is the same one.  With one
+        // right-hand side the last wavefronts publish and the first ones read:
+        // loads behind a store wait for its acknowledgement, one counter
+        // serves both (with three all of them read).
+        auto group_total = [&](double t, int id) {
+            // lane's value is group id's sum: the four in pairs
+            static_assert(NGRP == 4, "two pairs");
+            int at[NGRP];
+#pragma unroll
+            for (int g = 0; g < NGRP; g++) at[g] = __builtin_ctzll(__ballot(id == g));
+            return (lane_at(t, at[0]) + lane_at(t, at[1])) + (lane_at(t, at[2]) + lane_at(t, at[3]));
+        };
+        double own_total = 0.;   // a team of one: value `lane`
         auto collect = [&](int nv, uint32_t seq, uint32_t hseq) {
             TeamPtr A = team_args();
-            const bool mine = hseq != 0 && tid < H;
+            const bool mine = hseq != 0 && tid < H, rows_too = __any(mine);
             TeamWait w;
             bool ok = true;
             if (G == 1) {
                 // the tiles are here: the butterfly over at most 16 lanes that
-                // hold one, by one lane a value
-                if (wave == 0 && lane < nv) {
-                    double t[16];
+                // hold one, by one lane a value; every wavefront for itself,
+                // so that no barrier follows
+                if (lane < nv) {
+                    double t[MAXT];
 #pragma unroll
-                    for (int i = 0; i < 16; i++) t[i] = i < MAXT && i < mytiles ? 0. + tile_sum(i, lane) : 0.;
+                    for (int i = 0; i < MAXT; i++) t[i] = i < mytiles ? 0. + tile_sum(i, lane) : 0.;
 #pragma unroll
-                    for (int h = 8; h > 0; h >>= 1)
+                    for (int h = MAXT / 2; h > 0; h >>= 1)   // (0. + t is not -0.: the zeros beyond change nothing)
 #pragma unroll
                         for (int i = 0; i < h; i++) t[i] += t[i + h];
-                    red[lane] = t[0];
+                    red[lane] = own_total = t[0];
                 }
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 return;
             }
             if (!hop) {
-                // one right-hand side has few values: wavefront 0 reads them all
-                constexpr int N = NR == 1 ? NVC : MAXV, STEP = NR == 1 ? 1 : TEAM_WAVES;
-                const int v0 = NR == 1 ? 0 : wave;
-                const bool in = lane < mb.ntiles && (NR > 1 || wave == 0);
-                double s[N];
-                const uint64_t *x0 = xb_at(seq, v0, lane);
+                // wavefront w reads values w, w + 8, ...
+                double s[MAXV][NDIR];
                 for (;;) {
                     bool all = true;
+                    TeamWord<double> w1[MAXV][NDIR];
+                    Row row;
+                    auto reads = [&](int i, int g) {
+                        return wave + i * TEAM_WAVES < nv && g * WAVE < mb.ntiles;
+                    };
 #pragma unroll
-                    for (int i = 0; i < N; i++) {
-                        s[i] = 0.;
-                        if (in && v0 + i * STEP < nv) {
-                            all &= poll_sum(x0 + (size_t)(i * STEP * mb.ntiles) * 2, seq, s[i]);
-                            s[i] = 0. + s[i];
+                    for (int i = 0; i < MAXV; i++)
+#pragma unroll
+                        for (int g = 0; g < NDIR; g++)
+                            if (NDIR == 1 || reads(i, g)) {   // (one group: value nv - 1 again, no branch)
+                                const uint64_t *o = xb_at(seq, min(wave + i * TEAM_WAVES, nv - 1),
+                                                          min(g * WAVE + lane, mb.ntiles - 1));
+                                w1[i][g].load(o, o + 1, 0);
+                            }
+                    if (rows_too) row.load(A, hseq, halo_row);
+#pragma unroll
+                    for (int i = 0; i < MAXV; i++)
+#pragma unroll
+                        for (int g = 0; g < NDIR; g++) {
+                            s[i][g] = 0.;
+                            if (NDIR == 1 || reads(i, g)) {
+                                all &= w1[i][g].is(seq);
+                                if (g * WAVE + lane < mb.ntiles) s[i][g] = 0. + w1[i][g].value();
+                            }
                         }
-                    }
-                    if (mine) all &= poll_row(A, hseq, halo_row, hv);
+                    if (rows_too) all &= row.get(hseq, hv) || !mine;
                     if (__all(all)) break;
                     if (!w.again(A->t.ctl)) { ok = false; break; }
                 }
-                if (NR > 1 || wave == 0) {
+                if constexpr (NDIR == 1) {
                     int id;
-                    const double tot = wave_sums<N>(s, lane, id);
-                    if ((lane & 1) == 0 && v0 + id * STEP < nv) red[v0 + id * STEP] = tot;
+                    double sv[MAXV];
+#pragma unroll
+                    for (int i = 0; i < MAXV; i++) sv[i] = s[i][0];
+                    const double tot = wave_sums<MAXV>(sv, lane, id);
+                    const int v = wave + id * TEAM_WAVES;
+                    if ((lane & 1) == 0 && v < nv) red[v] = tot;
+                } else {
+                    static_assert(MAXV == 1, "one value a wavefront");
+                    const int v = wave;
+                    if (v < nv) {
+                        // (the columns beyond the tiles are zeros: sums of
+                        // empty groups are 0. and adding them changes nothing)
+                        int id;
+                        double tot;
+                        if (mb.ntiles <= WAVE) {
+                            tot = wave_sums<1>(s[0], lane, id);
+                        } else {
+                            const double t = wave_sums<NDIR>(s[0], lane, id);
+                            tot = group_total(t, id);
+                        }
+                        if (lane == 0) red[v] = tot;
+                    }
                 }
                 if (!ok) s_bad = 1;
-                if (NR > 1) __syncthreads();
-                else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __syncthreads();
                 return;
             }
             // four wavefronts sum a value
@@ -580,11 +720,18 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                         double c[Q];
                         for (;;) {
                             bool all = true;
+                            TeamWord<double> wu[Q];
+#pragma unroll
+                            for (int u = 0; u < Q; u++)
+                                if (u0 + u < nu) {
+                                    const uint64_t *o = xb_at(seq, v, min((u0 + u) * TEAM_COLS + g * WAVE + lane, mb.ntiles - 1));
+                                    wu[u].load(o, o + 1, 0);
+                                }
 #pragma unroll
                             for (int u = 0; u < Q; u++) {
-                                const int t = (u0 + u) * TEAM_COLS + g * WAVE + lane;
-                                c[u] = 0.;
-                                if (u0 + u < nu && t < mb.ntiles) all &= poll_sum(xb_at(seq, v, t), seq, c[u]);
+                                const bool use = u0 + u < nu && (u0 + u) * TEAM_COLS + g * WAVE + lane < mb.ntiles;
+                                all &= wu[u].is(seq) || !use;
+                                c[u] = use ? wu[u].value() : 0.;
                             }
                             if (__all(all)) break;
                             if (!w.again(A->t.ctl)) { ok = false; break; }
@@ -598,23 +745,27 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                 const double tot = wave_sums<1>(&s, lane, id);
                 if (lane == 0) grp[half][g] = tot;
                 __syncthreads();
-                if (lane == 0 && g == 0 && v < nv)
+                if (lane == 0 && g == (NR == 1 ? NGRP - 1 : 0) && v < nv)
                     put_sum(total_at(seq, v), (grp[half][0] + grp[half][1]) + (grp[half][2] + grp[half][3]), seq);
                 if (v0 + HALVES * G < nv) __syncthreads();
             }
             for (;;) {
                 bool all = true;
-                if (wave == 0 && lane < nv) {
-                    double s;
-                    all &= poll_sum(total_at(seq, lane), seq, s);
-                    red[lane] = s;
+                const uint64_t *o = total_at(seq, lane < nv ? lane : 0);
+                TeamWord<double> tot;
+                Row row;
+                if (wave == 0) tot.load(o, o + 1, 0);
+                if (rows_too) row.load(A, hseq, halo_row);
+                if (wave == 0) {
+                    all &= tot.is(seq) || lane >= nv;
+                    if (lane < nv) red[lane] = tot.value();
                 }
-                if (mine) all &= poll_row(A, hseq, halo_row, hv);
+                if (rows_too) all &= row.get(hseq, hv) || !mine;
                 if (__all(all)) break;
                 if (!w.again(A->t.ctl)) { ok = false; break; }
             }
             if (!ok) s_bad = 1;
-            if (wave == 0) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __syncthreads();
         };
         // Words of q (or r) of the exported row of slice j.
         auto export_row = [&](int j, int row, W(*v)[B], uint32_t seq) {
@@ -818,19 +969,52 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
         };
         if (!s_bad) refine(true);
 
-        typedef TeamGroup<M, B, NR> Group;
+        // streamed groups: 16-37 registers, twice (the next group is loaded
+        // while one is multiplied); beside resident blocks once
+        constexpr int R = team_resident<M, B, NR, J>();
+        constexpr int N = R > 0 ? 2 : (std::is_same<M, Dict>::value ? 8 : (B * NR == 2 ? 4 : 2));
+        typedef TeamGroup<M, B, N> Group;
+        TeamRes<M, B, R> res[J];
         Group cur;
         {
-            const Slice sl = first_slice;
             TeamPtr A = team_args();
-            cur.load(A->t.lidx, A->a.vw, A->a.nslots, sl.s0, sl.width, lane);
+#pragma unroll
+            for (int j = 0; j < J; j++) {
+                const Slice sl = slice_of(j);
+                res[j].load(A->t.lidx, A->a.vw, A->a.nslots, sl.s0, sl.width, lane);
+            }
+            if (R == 0) {
+                const Slice sl = first_slice;
+                cur.load(A->t.lidx, A->a.vw, A->a.nslots, sl.s0, sl.width, lane);
+            }
         }
+        // What the quick iterations know of the problem's record; lane k of
+        // each wavefront has right-hand side k.
+        int dmask;
+        int64_t iters, due;
+        double rr_need;
+        bool pending, refined = true;   // refined: the latest residual sums are a refinement's
+        auto quick_state = [&] {
+            const int k = lane < NR ? lane : NR - 1;
+            dmask = 0;
+            for (int i = 0; i < NR; i++) dmask |= (P.done[i] ? 1 : 0) << i;
+            iters = P.iters;
+            due = P.maxit - P.last_ckpt < P.ckpt_interval ? P.maxit : P.last_ckpt + P.ckpt_interval;
+            // rr < drop, or rr <= target
+            const double drop = P.drop * P.drop * P.rr_ckpt[k];
+            const double below = drop > 0. ? __longlong_as_double(__double_as_longlong(drop) - 1) : -1.;
+            rr_need = fmax(below, P.rr_target[k]);
+            pending = P.ckpt_pending != 0;
+        };
+        __syncthreads();
+        quick_state();
         int period = 0;
         const int ce = A0->t.ce, max_periods = A0->t.max_periods;
         while (!s_bad && period < max_periods) {
             bool running = true;
             for (int it = 0; it < ce && running; it++) {
                 // ---- K1: q = Ks p, sums of p.q, q.z, q.Mq
+                fresh();
                 qs++;
                 TeamPtr A = team_args();
                 const uint16_t *lidx = A->t.lidx;
@@ -847,32 +1031,50 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                     for (int k = 0; k < NR; k++)
 #pragma unroll
                         for (int i = 0; i < B; i++) acc[k][i] = 0.;
-                    // one group at least (an absent slice's is null), and
-                    // while it is multiplied the next one's loads: of this
-                    // slice, of the next, or of the first in the next
-                    // iteration (its wait is then the exchange's)
+                    auto block = [&](uint32_t li, const TeamBlk<M, B> &blk) {
+                        W tv[NR][B];
+                        rec_load<W, B, NR>(lp + REC * li, tv);
+#pragma unroll
+                        for (int jj = 0; jj < B; jj++)
+#pragma unroll
+                            for (int i = 0; i < B; i++) {
+                                const double m = blk.at(tab, jj * B + i);
+#pragma unroll
+                                for (int k = 0; k < NR; k++) acc[k][i] = mac(m, (double)tv[k][jj], acc[k][i]);
+                            }
+                    };
                     int kb = 0;
-                    do {
-                        Group next;
-                        kb += Group::N;
-                        const bool more = kb < sl.width;
-                        next.load(lidx, vw_, ns, more ? sl.s0 + (int64_t)kb * WAVE : after.s0,
-                                  more ? sl.width - kb : after.width, lane);
+                    if constexpr (R > 0) {
+                        if (R < sl.width) cur.load(lidx, vw_, ns, sl.s0 + R * WAVE, sl.width - R, lane);
 #pragma unroll
-                        for (int u = 0; u < Group::N; u++) {
-                            W tv[NR][B];
-                            rec_load<W, B, NR>(lp + REC * cur.li[u], tv);
+                        for (; kb < R; kb += 4)
+                            if (kb < sl.width) {
+                                res[j].keep(kb);
 #pragma unroll
-                            for (int jj = 0; jj < B; jj++)
+                                for (int u = 0; u < 4; u++) block(res[j].col(kb + u), res[j].blk[kb + u]);
+                            }
+                        while (kb < sl.width) {
 #pragma unroll
-                                for (int i = 0; i < B; i++) {
-                                    const double m = cur.blk[u].at(tab, jj * B + i);
-#pragma unroll
-                                    for (int k = 0; k < NR; k++) acc[k][i] = mac(m, (double)tv[k][jj], acc[k][i]);
-                                }
+                            for (int u = 0; u < N; u++) block(cur.li[u], cur.blk[u]);
+                            kb += N;
+                            if (kb < sl.width) cur.load(lidx, vw_, ns, sl.s0 + (int64_t)kb * WAVE, sl.width - kb, lane);
                         }
-                        cur = next;
-                    } while (kb < sl.width);
+                    } else {
+                        // one group at least (an absent slice's is null), and
+                        // while it is multiplied the next one's loads: of this
+                        // slice, of the next, or of the first in the next
+                        // iteration (its wait is then the exchange's)
+                        do {
+                            Group next;
+                            kb += N;
+                            const bool more = kb < sl.width;
+                            next.load(lidx, vw_, ns, more ? sl.s0 + (int64_t)kb * WAVE : after.s0,
+                                      more ? sl.width - kb : after.width, lane);
+#pragma unroll
+                            for (int u = 0; u < N; u++) block(cur.li[u], cur.blk[u]);
+                            cur = next;
+                        } while (kb < sl.width);
+                    }
                     double v[3 * NR];
 #pragma unroll
                     for (int i = 0; i < 3 * NR; i++) v[i] = 0.;
@@ -903,35 +1105,77 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                 xs++;
                 publish(0, 3 * NR, xs);
                 // ---- R: the same scalars in every member
-                const bool ck = P.src_ckpt != 0;
+                fresh();
+                double al64[NR];
+                W be[NR];
+                bool slot = false;
+                const bool ck = refined;
+                refined = false;
                 collect(ck ? NVC : NVN, xs, G > 1 ? qs : 0);
-                if (wave == 0) {
-                    int f = 0;
-                    if (lane < NR) {
-                        const int k = lane;
-                        f = reduce_rhs(P, k, red[k], red[NR + k], red[2 * NR + k], red[3 * NR + k],
-                                       red[3 * NR + NRES - NR + k], ck ? red[NVN + k] : 0., ck ? red[NVN + NR + k] : 0.,
-                                       ck);
+                // An iteration in the middle of a period needs alpha and
+                // beta, which every wavefront forms for itself, and whether a
+                // refinement is due or something went wrong (reduce_rhs and
+                // reduce_finish without their records: those cost 1800
+                // cycles on the way from the sums to the update, this 500).
+                bool quick = !ck && it != ce - 1;
+                if (quick) {
+                    const int k = lane < NR ? lane : NR - 1;
+                    auto sum_of = [&](int v) { return NR == 1 && G == 1 ? lane_value(own_total, v) : red[v + k]; };
+                    const double pq = sum_of(0), qz = sum_of(NR), qmq = sum_of(2 * NR), rho = sum_of(3 * NR),
+                                 rr = sum_of(3 * NR + NRES - NR);
+                    const bool dn = dmask >> k & 1;
+                    const double alpha = dn ? 0. : (pq != 0. ? rho / pq : 0.);
+                    const double rho1 = mac(alpha * alpha, qmq, mac(-2. * alpha, qz, rho));
+                    const double beta = dn ? 0. : (rho != 0. ? rho1 / rho : 0.);
+                    quick = !__any(!dn && (!(pq == pq) || !(rho == rho) || !(qz == qz) || !(qmq == qmq)));
+                    if (quick) {
+                        if (wave == 0 && lane < NR && !dn) P.rho_pred[k] = rho1;   // read by the next refinement's
+                        iters++;
+                        if (__any(!dn && rr <= rr_need) || iters >= due) pending = true;
+#pragma unroll
+                        for (int kk = 0; kk < NR; kk++) {
+                            al64[kk] = NR == 1 ? alpha : lane_value(alpha, kk);
+                            be[kk] = (W)(NR == 1 ? beta : lane_value(beta, kk));
+                        }
                     }
-                    for (int k = 1; k < NR; k++) f |= __shfl(f, k, WAVE);
-                    if (lane == 0) reduce_finish(P, f, ck);
                 }
-                __syncthreads();
-                if (s_bad) break;
-                running = P.status == ST_RUNNING;
-                if (!running) break;
+                if (!quick) {
+                    if (wave == 0) {
+                        int f = 0;
+                        if (lane == 0) {   // as the quick iterations left them
+                            P.iters = iters;
+                            if (pending) P.ckpt_pending = 1;
+                        }
+                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                        if (lane < NR) {
+                            const int k = lane;
+                            f = reduce_rhs(P, k, red[k], red[NR + k], red[2 * NR + k], red[3 * NR + k],
+                                           red[3 * NR + NRES - NR + k], ck ? red[NVN + k] : 0., ck ? red[NVN + NR + k] : 0.,
+                                           ck);
+                        }
+                        for (int k = 1; k < NR; k++) f |= __shfl(f, k, WAVE);
+                        if (lane == 0) reduce_finish(P, f, ck);
+                    }
+                    __syncthreads();
+                    if (s_bad) break;
+                    running = P.status == ST_RUNNING;
+                    if (!running) break;
+                    slot = it == ce - 1 && P.ckpt_pending;
+                    quick_state();
+#pragma unroll
+                    for (int k = 0; k < NR; k++) {
+                        al64[k] = P.alpha[k];
+                        be[k] = (W)P.beta[k];
+                    }
+                }
+                fresh();
                 // ---- K2: y, r, p of the own rows and of the halo.  A
                 // finished right-hand side has alpha = beta = 0: its y and r
                 // stay as they are, and its p feeds nothing any more.
-                const bool slot = it == ce - 1 && P.ckpt_pending;
-                double al64[NR];
-                W al[NR], be[NR];
+                W al[NR];
 #pragma unroll
-                for (int k = 0; k < NR; k++) {
-                    al64[k] = P.alpha[k];
-                    al[k] = (W)al64[k];
-                    be[k] = (W)P.beta[k];
-                }
+                for (int k = 0; k < NR; k++) al[k] = (W)al64[k];
+                rp ^= 1;
                 auto k2_row = [&](W(*pk)[B], W(*rk)[B], const W(*qk)[B], const W *mi, auto each) {
 #pragma unroll
                     for (int k = 0; k < NR; k++) {
@@ -988,13 +1232,16 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                 __syncthreads();
                 if (!slot) publish(3 * NR, NVN, xs + 1);
                 else if (tid == 0) P.src_ckpt = 1;
-                if (s_bad) break;
+                if (it == ce - 1 && s_bad) break;   // (a wait that gave up: the quick iterations do not look)
             }
             if (!running || s_bad) break;
             period++;
             if (mb.m == 0 && tid == 0)
                 __hip_atomic_fetch_add(team_args()->t.ctl + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (P.ckpt_pending) refine(false);
+            if (P.ckpt_pending) {
+                refine(false);
+                refined = true;
+            }
         }
         seq_max = seq_max > xs ? seq_max : xs;
         seq_max = seq_max > qs ? seq_max : qs;
