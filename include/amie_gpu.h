@@ -134,10 +134,11 @@ typedef struct {
     int32_t persistent;      /* > 0: AMIE_FP64 and AMIE_MIXED_FIX48 run each solve pass as one
                                 persistent launch of at most this many workgroups (all resident),
                                 the iteration phases separated by device-wide barriers instead of
-                                kernel boundaries; the same results bit for bit.  For small
-                                batches and served groups: a barrier's cost grows with the
-                                workgroups (about 2-3 us at 64).  0 (default): one launch per
-                                phase. */
+                                kernel boundaries; the same results bit for bit.  0 (default):
+                                AMIE_FP64 and AMIE_MIXED_FIX48 run a pass as one launch whose
+                                workgroups keep their rows on the chip, unless time_kernels or
+                                use_graph asks for kernels (again the same results bit for bit);
+                                the other precisions one launch per phase. */
 } amie_solve_opts;
 
 typedef struct {
@@ -465,14 +466,10 @@ int amie_gpu_batch_set_damage(amie_gpu_batch *b, int32_t p, const double *d);
  * neighbourhood (FractureCriterion::getMaxScoreInNeighbourhood,
  * fracturecriterion.cpp:251-280) takes d += fibre_fraction } until a pass
  * changes nothing.  Linear elements (P1, Tet4), right-hand side 0.  With
- * opts.persistent 0 the solves take shorter-latency paths, in FP64
- * whatever opts.precision asks (same stopping rule: FP64 relative residual
- * <= opts.rtol), for one right-hand side: each problem's whole CG in one
- * workgroup when every problem has at most 3 072 block rows (2 048 for
- * Tet4), or a batch of one problem of at most 131 072 block rows over a
- * cooperative grid of up to 64 workgroups; otherwise a batch of at most 32
- * tiles (8 192 block rows) solves with persistent launches (the launch
- * path's results bit for bit). */
+ * opts.persistent 0 small meshes solve in FP64 whatever opts.precision asks
+ * (same stopping rule: FP64 relative residual <= opts.rtol), for one
+ * right-hand side: a batch whose problems have at most 3 072 block rows each
+ * (2 048 for Tet4), or a batch of one problem of at most 131 072. */
 typedef struct {
     int32_t nphase;              /* materials the two arrays below cover (>= every problem's nphase) */
     const int32_t *criterion;    /* per material: 1 = StiffnessAndFracture + NonLocalMazars, 0 = elastic */

@@ -992,7 +992,7 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
         // each wavefront has right-hand side k.
         int dmask;
         int64_t iters, due;
-        double rr_need;
+        double rr_need, rho_keep = 0.;
         bool pending, refined = true;   // refined: the latest residual sums are a refinement's
         auto quick_state = [&] {
             const int k = lane < NR ? lane : NR - 1;
@@ -1112,12 +1112,13 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                 const bool ck = refined;
                 refined = false;
                 collect(ck ? NVC : NVN, xs, G > 1 ? qs : 0);
-                // An iteration in the middle of a period needs alpha and
-                // beta, which every wavefront forms for itself, and whether a
+                // Most iterations need alpha and beta, which every wavefront forms for itself, and whether a
                 // refinement is due or something went wrong (reduce_rhs and
                 // reduce_finish without their records: those cost 1800
                 // cycles on the way from the sums to the update, this 500).
-                bool quick = !ck && it != ce - 1;
+                // (With more slices a wavefront the registers for a period's last
+                // iteration are not there.)
+                bool quick = !ck && (J == 1 || it != ce - 1);
                 if (quick) {
                     const int k = lane < NR ? lane : NR - 1;
                     auto sum_of = [&](int v) { return NR == 1 && G == 1 ? lane_value(own_total, v) : red[v + k]; };
@@ -1128,10 +1129,17 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                     const double rho1 = mac(alpha * alpha, qmq, mac(-2. * alpha, qz, rho));
                     const double beta = dn ? 0. : (rho != 0. ? rho1 / rho : 0.);
                     quick = !__any(!dn && (!(pq == pq) || !(rho == rho) || !(qz == qz) || !(qmq == qmq)));
+                    bool due_now = false;
+                    if constexpr (J == 1) {
+                        due_now = pending || __any(!dn && rr <= rr_need) || iters + 1 >= due;
+                        quick = quick && !(due_now && it == ce - 1);   // the refinement's slot
+                    }
                     if (quick) {
-                        if (wave == 0 && lane < NR && !dn) P.rho_pred[k] = rho1;   // read by the next refinement's
+                        if constexpr (J == 1) rho_keep = rho1;
+                        else if (wave == 0 && lane < NR && !dn) P.rho_pred[k] = rho1;   // for the next refinement's
                         iters++;
-                        if (__any(!dn && rr <= rr_need) || iters >= due) pending = true;
+                        if constexpr (J == 1) pending = due_now;
+                        else if (__any(!dn && rr <= rr_need) || iters >= due) pending = true;
 #pragma unroll
                         for (int kk = 0; kk < NR; kk++) {
                             al64[kk] = NR == 1 ? alpha : lane_value(alpha, kk);
@@ -1142,7 +1150,8 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                 if (!quick) {
                     if (wave == 0) {
                         int f = 0;
-                        if (lane == 0) {   // as the quick iterations left them
+                        if (J == 1 && lane < NR && iters != P.iters && !P.done[lane]) P.rho_pred[lane] = rho_keep;
+                        if (lane == 0) {   // as
                             P.iters = iters;
                             if (pending) P.ckpt_pending = 1;
                         }
@@ -1245,6 +1254,7 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
         }
         seq_max = seq_max > xs ? seq_max : xs;
         seq_max = seq_max > qs ? seq_max : qs;
+        if (J == 1 && tid == 0 && !s_bad) P.iters = iters;
         __syncthreads();
         if (mb.m == 0 && !s_bad)
             for (int i = tid; i < (int)(sizeof(ProbDev) / 4); i += TEAM_WG)
