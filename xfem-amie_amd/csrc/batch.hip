@@ -1942,17 +1942,26 @@ int amie_gpu_batch_average_stress(amie_gpu_batch *bb, double *outp)
     if (!B.has_elements) { set_error("batch has no elements"); return AMIE_ERR_STATE; }
     DevBuf out;
     const size_t n = (size_t)B.nprob * B.nrhs * B.et.s;
-    if (!out.alloc(n * 8)) return AMIE_ERR_NOMEM;
+    int64_t ne = 1;
+    for (const ProbHost &P : B.ph) ne = std::max<int64_t>(ne, P.nelem);
+    const unsigned nchunk = (unsigned)((ne + AVG_CHUNK - 1) / AVG_CHUNK);
+    const size_t npart = (size_t)(B.nelem / AVG_CHUNK + B.nprob + 1) * B.nrhs * (B.et.s + 1);
+    if (!out.alloc((n + npart) * 8)) return AMIE_ERR_NOMEM;
+    double *part = out.as<double>() + n;
     StrainArgs s = strain_args(B);
     hipStream_t st = B.stream;
-    auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(B.nprob), dim3(256), 0, st, s, B.prob_e0.as<int32_t>(), B.prob_ne.as<int32_t>(),
-                           B.ephase.as<int32_t>(), B.edamage.as<double>(), B.cmat_off.as<int32_t>(), B.cmat.as<double>(),
-                           out.as<double>(), B.frac_at, B.frac_residual);
+    auto go = [&](auto kern, auto final_kern) {
+        for (int p0 = 0; p0 < B.nprob; p0 += 65535)   // problems in the grid's y
+            hipLaunchKernelGGL(kern, dim3(nchunk, (unsigned)std::min(65535, B.nprob - p0), B.nrhs), dim3(256), 0, st, s,
+                               B.prob_e0.as<int32_t>(), B.prob_ne.as<int32_t>(), B.ephase.as<int32_t>(),
+                               B.edamage.as<double>(), B.cmat_off.as<int32_t>(), B.cmat.as<double>(), part, B.frac_at,
+                               B.frac_residual, p0);
+        hipLaunchKernelGGL(final_kern, dim3(B.nprob * B.nrhs), dim3(WAVE), 0, st, part, B.prob_e0.as<int32_t>(),
+                           B.prob_ne.as<int32_t>(), B.nrhs, out.as<double>());
     };
-    if (B.et.et == 1) go(k_average_stress<1>);
-    else if (B.et.et == 2) go(k_average_stress<2>);
-    else go(k_average_stress<3>);
+    if (B.et.et == 1) go(k_average_stress<1>, k_average_final<3>);
+    else if (B.et.et == 2) go(k_average_stress<2>, k_average_final<3>);
+    else go(k_average_stress<3>, k_average_final<6>);
     AMIE_HIP(hipGetLastError());
     AMIE_HIP(hipStreamSynchronize(st));
     AMIE_HIP(hipMemcpy(outp, out.p, n * 8, hipMemcpyDeviceToHost));
