@@ -853,8 +853,9 @@ __global__ __launch_bounds__(256) void k_smooth(NonlocalArgs a, const double *st
                 const int cell = gd[3] + (z * gd[1] + y) * gd[0] + x;
                 for (int j = a.cell_start[cell] + lane; j < a.cell_start[cell + 1]; j += LANES) {
                     const int i = a.cell_elem[j];
-                    if (a.ephase && a.ephase[i] != ph) continue;
-                    if (a.edamage && a.edamage[i] >= a.threshold) continue;
+                    // five of six candidates are too far: their phase and
+                    // damage are not loaded (Tet4 24^3, 83 000 elements:
+                    // 6.7 -> 6.2 ms)
                     const double *gi = a.geo + (int64_t)i * GEO_STRIDE;
                     double d2 = 0.;
                     for (int d = 0; d < D; d++) d2 += (gi[d] - c[d]) * (gi[d] - c[d]);
@@ -862,6 +863,8 @@ __global__ __launch_bounds__(256) void k_smooth(NonlocalArgs a, const double *st
                     // with its 1e-12 tolerance (geometry_3D.cpp:1551-1566)
                     const bool in = D == 2 ? d2 < rho * rho : d2 < rho * rho + 2. * rho * 1e-12 + 1e-24;
                     if (!in) continue;
+                    if (a.ephase && a.ephase[i] != ph) continue;
+                    if (a.edamage && a.edamage[i] >= a.threshold) continue;
                     double coef = 0.;
                     for (int v = 0; v < NP; v++) {
                         const int nd = a.econn[(int64_t)i * NP + v];
