@@ -413,6 +413,24 @@ int amie_gpu_batch_autotune(amie_gpu_batch *b, int32_t precision, int32_t precon
  * (AMIE_ERR_ARG otherwise).  No reference counterpart. */
 int amie_gpu_batch_set_spmv_kernel(amie_gpu_batch *b, int32_t precision, int32_t precond, int32_t steps,
                                    int32_t tile_order, int32_t format);
+/* How the AMIE_FP64 and AMIE_MIXED_FIX48 passes of this batch run where
+ * neither time_kernels, persistent nor use_graph says it: AUTO (the default)
+ * leaves it to the library; ALWAYS takes the one launch that keeps the rows
+ * on the chip wherever the batch fits it, NEVER one launch per phase.  The
+ * results are the same bits.  tiles > 0 sets the tiles (of 256 block rows)
+ * a workgroup holds in the one launch, 0 leaves them to the library.  No
+ * reference counterpart. */
+enum { AMIE_TEAM_AUTO = 0, AMIE_TEAM_ALWAYS = 1, AMIE_TEAM_NEVER = 2 };
+int amie_gpu_batch_set_team(amie_gpu_batch *b, int32_t use, int32_t tiles);
+/* How the latest solve of this batch ran. */
+typedef struct {
+    int32_t passes;          /* solve passes */
+    int32_t team_passes;     /* of them as one launch */
+    int32_t tiles;           /* most tiles a workgroup held in the latest such launch */
+    int32_t workgroups;      /* that its problems were cut into */
+    int64_t halo_rows;       /* rows of other workgroups that these keep a copy of, summed */
+} amie_team_info;
+int amie_gpu_batch_team_info(amie_gpu_batch *b, amie_team_info *info);
 /* Element strains (nelem x 3|6, Voigt, engineering shear) of right-hand side
  * rhs, including the macro strain. */
 int amie_gpu_batch_element_strain(amie_gpu_batch *b, int32_t p, int32_t rhs, double *strain);

@@ -17,6 +17,7 @@ FP64, MIXED, MIXED64, MIXED_K64, MIXED_SPLIT, MIXED_FIX48 = 0, 1, 2, 3, 4, 5
 DAMAGE_FIBRE, DAMAGE_ISOTROPIC_LINEAR = 0, 1   # event-damage models (amie_event_params.damage_model)
 JACOBI, BLOCK_JACOBI = 0, 1
 REFINE_REPLACE, REFINE_RESTART = 0, 1
+TEAM_AUTO, TEAM_ALWAYS, TEAM_NEVER = 0, 1, 2
 ASSEMBLE_GATHER, ASSEMBLE_COLOURED = 0, 1
 NPER = {P1: 3, P2: 6, TET4: 4}
 DIM = {P1: 2, P2: 2, TET4: 3}
@@ -66,6 +67,14 @@ class EventParams(ctypes.Structure):
 class EventStats(ctypes.Structure):
     _fields_ = [("passes", c_i64), ("cg_iterations", c_i64), ("events", c_i64), ("fractured", c_i64),
                 ("status", c_i32), ("converged", c_i32), ("solve_ms", c_dbl), ("damage_ms", c_dbl)]
+
+    def as_dict(self):
+        return {k: getattr(self, k) for k, _ in self._fields_}
+
+
+class TeamInfo(ctypes.Structure):
+    _fields_ = [("passes", c_i32), ("team_passes", c_i32), ("tiles", c_i32), ("workgroups", c_i32),
+                ("halo_rows", c_i64)]
 
     def as_dict(self):
         return {k: getattr(self, k) for k, _ in self._fields_}
@@ -126,6 +135,8 @@ SIGNATURES = {
     "amie_gpu_batch_set_nonlocal": (c_i32, [vp, c_dbl, c_i32, c_dbl]),
     "amie_gpu_batch_smoothed_strain": (c_i32, [vp, c_i32, c_i32, vp]),
     "amie_gpu_batch_set_spmv_kernel": (c_i32, [vp, c_i32, c_i32, c_i32, c_i32, c_i32]),
+    "amie_gpu_batch_set_team": (c_i32, [vp, c_i32, c_i32]),
+    "amie_gpu_batch_team_info": (c_i32, [vp, vp]),
     "amie_gpu_batch_element_strain": (c_i32, [vp, c_i32, c_i32, vp]),
     "amie_gpu_batch_average_stress": (c_i32, [vp, vp]),
     "amie_gpu_batch_damage_step": (c_i32, [vp, vp, vp]),
@@ -575,6 +586,16 @@ class Batch:
         """Selects an SpMV candidate directly (blocks per step, tile order,
         format 0 value planes / 1 value-indexed FIX48 matrix)."""
         check(lib().amie_gpu_batch_set_spmv_kernel(self.h, precision, precond, steps, tile_order, format))
+
+    def set_team(self, use=TEAM_AUTO, tiles=0):
+        """Whether FP64 and FIX48 passes run as one launch (TEAM_AUTO,
+        TEAM_ALWAYS, TEAM_NEVER) and the tiles a workgroup holds in it."""
+        check(lib().amie_gpu_batch_set_team(self.h, use, tiles))
+
+    def team_info(self):
+        info = TeamInfo()
+        check(lib().amie_gpu_batch_team_info(self.h, ctypes.byref(info)))
+        return info.as_dict()
 
     def element_strain(self, p=0, rhs=0):
         pr = self.problems[p]

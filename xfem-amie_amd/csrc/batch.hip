@@ -1066,6 +1066,7 @@ int Batch::start_pass(int mode, const std::vector<char> &subset)
     }
     AMIE_HIP(hipMemcpyAsync(prob.p, h_prob.data(), nprob * sizeof(ProbDev), hipMemcpyHostToDevice, s));
     if (int rc = team_prepare(*this, R, subset)) return rc;
+    R.info.passes++;
     if (!R.team) {
         team_dirty = true;
         for (DevBuf *v : {&y, &p, &p2, &p3, &p4}) AMIE_HIP(hipMemsetAsync(v->p, 0, v->n, s));
@@ -1133,6 +1134,11 @@ int Batch::solve_advance()
         // the whole pass in one launch; the status copy follows it
         if (!R.persist_launched && R.team) {
             if (int rc = team_launch(*this, R)) return rc;
+            R.info.team_passes++;
+            R.info.tiles = R.team->tpw;
+            R.info.workgroups = (int32_t)R.team->h_order.size();
+            R.info.halo_rows = 0;
+            for (int32_t m : R.team->h_order) R.info.halo_rows += R.team->nhalo[m];
             R.persist_launched = true;
             R.periods = R.max_periods;
         } else if (!R.persist_launched) {
@@ -1869,6 +1875,26 @@ int amie_gpu_batch_set_spmv_kernel(amie_gpu_batch *bb, int32_t precision, int32_
     }
     set_error("no SpMV candidate with %d blocks per step for precision %d", steps, precision);
     return AMIE_ERR_ARG;
+}
+
+int amie_gpu_batch_set_team(amie_gpu_batch *bb, int32_t use, int32_t tiles)
+{
+    if (!bb || !bb->b || use < AMIE_TEAM_AUTO || use > AMIE_TEAM_NEVER || tiles < 0) {
+        set_error("bad arguments");
+        return AMIE_ERR_ARG;
+    }
+    Batch &B = *bb->b;
+    if (B.run.started) { set_error("a solve is in progress"); return AMIE_ERR_BUSY; }
+    B.team_use = use;
+    B.team_tiles = tiles;
+    return AMIE_OK;
+}
+
+int amie_gpu_batch_team_info(amie_gpu_batch *bb, amie_team_info *info)
+{
+    if (!bb || !bb->b || !info) { set_error("bad arguments"); return AMIE_ERR_ARG; }
+    *info = bb->b->run.info;
+    return AMIE_OK;
 }
 
 static StrainArgs strain_args(Batch &B)

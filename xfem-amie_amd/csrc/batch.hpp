@@ -81,6 +81,7 @@ struct TeamPlan {
     bool ok = false;                 // the problems fit
     int64_t lds_units = 0;           // largest member's own rows + 2 x halo rows
     std::vector<int32_t> first;      // per problem: its first member (one more at the end)
+    std::vector<int32_t> nhalo;      // per member: rows of others that it keeps
     std::vector<int32_t> h_order;    // members in the order they are claimed, as on the device
     DevBuf members, order, mslice, mtile, lidx, halo, exported, xb;
     size_t bytes() const
@@ -115,6 +116,7 @@ struct SolveRun {
     size_t team_lds = 0;             // its dynamic LDS
     bool team_single = false;        // every team is one workgroup
     bool persist_launched = false;   // either launch is queued
+    amie_team_info info{};
     amie_solve_stats stats{};
 };
 
@@ -197,6 +199,7 @@ struct Batch {
     std::vector<std::unique_ptr<TeamPlan>> team_plans;
     uint32_t team_seq = 0;                 // sequence numbers the team CG has used
     bool team_dirty = true;                // p2, p3, p4, y hold launch-path vectors
+    int team_use = AMIE_TEAM_AUTO, team_tiles = 0;   // amie_gpu_batch_set_team
 
     // captured iteration chunks, keyed by solve variant
     struct GraphEntry {

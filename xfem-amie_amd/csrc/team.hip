@@ -107,6 +107,10 @@ int team_tiles(const Batch &B, int jmax, double slot_bytes)
     for (const ProbHost &P : B.ph) big = std::max(big, P.ntiles);
     tpw = big <= 4 ? big : tpw;
     tpw = std::min(tpw, most);
+    if (B.team_tiles > 0) {
+        tpw = std::min(B.team_tiles, most);
+        return (big + tpw - 1) / tpw > cus ? 0 : tpw;
+    }
     auto members = [&](int t) {
         int64_t n = 0;
         for (const ProbHost &P : B.ph) n += (P.ntiles + t - 1) / t;
@@ -225,6 +229,7 @@ static int team_plan(Batch &B, int tpw, TeamPlan **out)
             T->lds_units = std::max<int64_t>(T->lds_units, rows + 2 * (int64_t)h[i]);
             if (rows + h[i] > 65536) T->ok = false;   // 16-bit local columns
         }
+        T->nhalo.swap(h);
         if (total >= INT32_MAX) T->ok = false;
         if (T->ok) {
             if (!T->halo.alloc((size_t)total * 4)) return no_room();
@@ -247,7 +252,8 @@ int team_prepare(Batch &B, SolveRun &R, const std::vector<char> &subset)
 {
     R.team = nullptr;
     const int mode = R.mode;
-    if ((mode != AMIE_FP64 && mode != AMIE_MIXED_FIX48) || R.o.time_kernels || R.o.persistent > 0 || R.o.use_graph)
+    if ((mode != AMIE_FP64 && mode != AMIE_MIXED_FIX48) || R.o.time_kernels || R.o.persistent > 0 || R.o.use_graph ||
+        B.team_use == AMIE_TEAM_NEVER)
         return AMIE_OK;
     const bool f64 = mode == AMIE_FP64;
     const int b = B.et.b, nr = B.nrhs, w = f64 ? 8 : 4;
