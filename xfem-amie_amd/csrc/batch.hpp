@@ -79,6 +79,9 @@ struct K1Choice {
 struct TeamPlan {
     int tpw = 0;                     // tiles per member
     bool ok = false;                 // the problems fit
+    int judged = -1;                 // precision and format the choice below was made for,
+    std::vector<int32_t> judged_probs;   // and problems
+    bool pays = true;                // a team launch is expected to be no slower than the launch path
     int64_t lds_units = 0;           // largest member's own rows + 2 x halo rows
     std::vector<int32_t> first;      // per problem: its first member (one more at the end)
     std::vector<int32_t> nhalo;      // per member: rows of others that it keeps
@@ -200,6 +203,7 @@ struct Batch {
     uint32_t team_seq = 0;                 // sequence numbers the team CG has used
     bool team_dirty = true;                // p2, p3, p4, y hold launch-path vectors
     int team_use = AMIE_TEAM_AUTO, team_tiles = 0;   // amie_gpu_batch_set_team
+    double team_margin = 1.;               // how much faster a team launch has to be expected
 
     // captured iteration chunks, keyed by solve variant
     struct GraphEntry {

@@ -122,6 +122,15 @@ struct Building {
     std::future<Built> fut;
 };
 
+// A group's team launch holds its CUs until the whole pass ends, and team
+// launches of several members run one after the other, while launches of the
+// iteration's phases interleave with the other groups'.  So it has to be
+// expected this much faster (served mix of 2D and 3D cells and damage steps,
+// 419 requests at 200 a second, solves/s with factors 1, 1.5, 2 and never: FP64
+// 52.9, 54.1, 52.5, 54.0, FIX48 95, 93, 82, 79; FP64 at 10 a second, median
+// latency 175, 108, 126, 136 ms).
+constexpr double TEAM_MARGIN = 1.5;
+
 template <typename T> static bool ready(std::future<T> &f)
 {
     return f.wait_for(std::chrono::seconds(0)) == std::future_status::ready;
@@ -390,6 +399,7 @@ struct Server {
                         return o;
                     }
                     o.rc = batch_create(cx, (int)descs.size(), descs.data(), &o.batch);
+                    if (o.rc == AMIE_OK) o.batch->team_margin = TEAM_MARGIN;
                     // the SpMV candidates are timed here too, off the serving thread
                     // (under the load of the groups in flight)
                     const bool tunable = so.precision == AMIE_FP64 || so.precision == AMIE_MIXED ||

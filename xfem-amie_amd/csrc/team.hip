@@ -1,6 +1,9 @@
 // Host side of the team CG (team.hpp): how a batch's problems are cut into
 // members, the halo plan, and the launch.
 #include <algorithm>
+#include <cmath>
+#include <functional>
+#include <queue>
 
 #include "batch.hpp"
 #include "team.hpp"
@@ -118,6 +121,103 @@ int team_tiles(const Batch &B, int jmax, double slot_bytes)
     };
     while (tpw < most && members(tpw) > cus) tpw++;
     return (big + tpw - 1) / tpw > cus ? 0 : tpw;
+}
+
+// The choice between the two paths, which give the same bits: estimated times
+// of a solve by each, in microseconds an iteration of a problem with a weight
+// of one.  Both follow what was measured (an MI355X, 205 batches of one to 64
+// problems by element, precision and right-hand sides, team and launches in
+// turn; the estimates' spread is about 10 %):
+//   launches   a floor of three dependent kernels and the stream of the matrix
+//              and the vectors at 4-6 TB/s, with a share a block for the
+//              value-indexed matrix.  They overlap where rows are long (3 x 3
+//              blocks) and add up where they are short.  A problem that is
+//              done leaves the iteration.
+//   team       a fixed part (sums, exchange, scalars), the product of the
+//              tiles a member holds, and the halo words of all members that
+//              run at a time, which come past the caches at 0.6-1 TB/s.
+//              Members are claimed in order, and a team whose last member has
+//              to wait for a CU keeps the others idle.
+// Almost everywhere the team is the faster one (1.1 to 6 times).  It is not
+// where teams of more than half the chip come one after the other (three
+// loads in FP64, a workgroup holds four tiles: 20 RVEs of 87..512 cells 357 us
+// an iteration against 277, two of 512 cells 95 against 88; but 64 of 36..256
+// cells 159 against 220) and where 3 x 3 blocks by value index read the table
+// for many slices in turn (12 RVEs of 19..48 cells: 101 against 76).
+struct Pace {
+    double fixed, tile[3];   // a tile with at most 2, 4 and 8 slices a wavefront
+};
+constexpr Pace PACE[3][2][2] = {   // FP64, FIX48 planes, value-indexed; 2 x 2, 3 x 3; one and three right-hand sides
+    {{{3.2, {0.3, 1.6, 1.6}}, {2.6, {1.9, 1.9, 1.9}}}, {{6.3, {0.3, 6.1, 6.1}}, {8.2, {5.2, 5.2, 5.2}}}},
+    {{{4.4, {0.3, 1.4, 1.4}}, {2.0, {1.8, 1.8, 1.8}}}, {{4.7, {2.2, 3.2, 6.1}}, {7.7, {4.5, 4.5, 4.5}}}},
+    {{{2.0, {0.7, 0.6, 0.7}}, {6.1, {0.3, 0.4, 0.4}}}, {{12.0, {0.4, 2.0, 5.3}}, {8.2, {4.8, 4.8, 4.8}}}},
+};
+// us a MB of halo words; a team of more than half the chip takes all of its
+// words at the same time, nothing between them
+constexpr double HALO_US_MB[2][2] = {{1.0, 1.25}, {1.75, 0.9}}, HALO_ALONE = 1.15;
+struct Launches {
+    double floor, tbs, block;   // us; TB/s; us per 10^6 value-indexed blocks
+};
+constexpr Launches LAUNCHES[2][2] = {{{16., 5.9, 1.8}, {23., 5.6, 2.9}}, {{24., 5.0, 6.0}, {32., 4.1, 8.6}}};
+
+// iterations of a problem, up to a factor: its nodes along one side
+double weight_of(const Batch &B, const ProbHost &P) { return std::pow((double)P.nrows, 1. / B.et.b); }
+
+double launch_estimate(const Batch &B, const std::vector<int32_t> &probs, bool f64, bool indexed)
+{
+    const int b = B.et.b, w = f64 ? 8 : 4;
+    const Launches &L = LAUNCHES[b - 2][B.nrhs > 1];
+    const double blocks = (double)B.nslots / std::max<double>(1., (double)B.nrows_pad) * WAVE * TILE_SLICES;   // a tile's
+    const double bytes = blocks * (indexed ? 4. : (f64 ? 8. : 6.) * b * b + 4.) +
+                         WAVE * TILE_SLICES * b * B.nrhs * (8.75 * w + 4.);
+    const double tile = bytes / L.tbs * 1e-6 + (indexed ? L.block * blocks * 1e-6 : 0.);
+    std::vector<std::pair<double, int>> by;   // the shortest solves end first
+    double active = 0., t = 0., done = 0.;
+    for (int p : probs) {
+        by.push_back({weight_of(B, B.ph[p]), B.ph[p].ntiles});
+        active += B.ph[p].ntiles;
+    }
+    std::sort(by.begin(), by.end());
+    for (auto &e : by) {
+        const double s = tile * active;
+        t += (e.first - done) * (b == 2 ? L.floor + s : std::hypot(L.floor, s));
+        done = e.first;
+        active -= e.second;
+    }
+    return t;
+}
+
+double team_estimate(const Batch &B, const TeamPlan &T, const std::vector<int32_t> &probs, bool f64, bool indexed, int j)
+{
+    const int b = B.et.b, nr = B.nrhs, cus = std::max(1, B.ctx->num_cu);
+    const Pace &C = PACE[f64 ? 0 : (indexed ? 2 : 1)][b - 2][nr > 1];
+    const double tile = C.tile[j <= 2 ? 0 : (j <= 4 ? 1 : 2)];
+    int64_t members = 0, halos = 0;
+    for (int p : probs) {
+        members += T.first[p + 1] - T.first[p];
+        for (int m = T.first[p]; m < T.first[p + 1]; m++) halos += T.nhalo[m];
+    }
+    const double us = HALO_US_MB[b - 2][nr > 1] * 8e-6 * b * nr * (f64 ? 2 : 1) * (double)std::min<int64_t>(members, cus);
+    const double mean = (double)halos / (double)std::max<int64_t>(1, members);
+    std::priority_queue<double, std::vector<double>, std::greater<double>> cu;   // when each is free
+    for (int i = 0; i < cus; i++) cu.push(0.);
+    double end = 0.;
+    for (int p : probs) {
+        const int G = T.first[p + 1] - T.first[p];
+        double halo = 0., from = 0.;
+        for (int m = T.first[p]; m < T.first[p + 1]; m++) halo += T.nhalo[m];
+        for (int m = 0; m < G; m++) {
+            from = std::max(from, cu.top());
+            cu.pop();
+        }
+        halo /= std::max(1, G);
+        if (b == 3) halo = 0.5 * (halo + mean);   // (other problems' halos are smaller)
+        const double to = from + weight_of(B, B.ph[p]) * (C.fixed + tile * std::min(T.tpw, B.ph[p].ntiles) +
+                                                          (2 * G > cus ? HALO_ALONE : 1.) * us * halo);
+        for (int m = 0; m < G; m++) cu.push(to);
+        end = std::max(end, to);
+    }
+    return end;
 }
 
 } // namespace
@@ -301,6 +401,19 @@ int team_prepare(Batch &B, SolveRun &R, const std::vector<char> &subset)
     for (int p : probs) {
         for (int m = T->first[p]; m < T->first[p + 1]; m++) order.push_back(m);
         single = single && T->first[p + 1] - T->first[p] == 1;
+    }
+    if (B.team_use == AMIE_TEAM_AUTO) {
+        const bool table = indexed && R.a.vw == B.dict_ids.p;
+        const int key = (f64 ? 1 : 0) | (indexed ? 2 : 0) | (table ? 4 : 0);
+        if (key != T->judged || probs != T->judged_probs) {
+            T->pays = B.team_margin * team_estimate(B, *T, probs, f64, table, j) <= launch_estimate(B, probs, f64, indexed);
+            T->judged = key;
+            T->judged_probs = probs;
+        }
+        if (!T->pays) {
+            if (indexed) R.a.vw = B.dict_ids.p;
+            return AMIE_OK;
+        }
     }
     if (order != T->h_order) {
         T->h_order.swap(order);   // kept: the source of the queued copy
