@@ -237,6 +237,9 @@ struct Batch {
 // The team CG: whether a pass runs as one (run.team), and its launch.
 int team_prepare(Batch &B, SolveRun &R, const std::vector<char> &subset);
 int team_launch(Batch &B, SolveRun &R);
+// Makes the plan that a solve with these options would make on its way, and
+// waits for it.
+int team_plan_ahead(Batch &B, const amie_solve_opts &o);
 
 // Builds the value-indexed FIX48 matrix of the current assembly (dict_ok
 // tells whether it exists: at most DICT_MAX distinct blocks).

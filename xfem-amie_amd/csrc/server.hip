@@ -406,6 +406,10 @@ struct Server {
                                          so.precision == AMIE_MIXED_FIX48;
                     if (o.rc == AMIE_OK && so.autotune && tunable)
                         o.rc = o.batch->autotune(so.precision, so.precond == AMIE_BLOCK_JACOBI, 3);
+                    // and the team plan is made: its allocations, host loops
+                    // and waits would hold the serving thread otherwise, and
+                    // its memory would not be in the group's bytes
+                    if (o.rc == AMIE_OK) o.rc = team_plan_ahead(*o.batch, so);
                     if (o.rc) {
                         o.err = amie_gpu_last_error();
                         delete o.batch;

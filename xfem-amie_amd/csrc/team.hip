@@ -426,6 +426,18 @@ int team_prepare(Batch &B, SolveRun &R, const std::vector<char> &subset)
     return AMIE_OK;
 }
 
+int team_plan_ahead(Batch &B, const amie_solve_opts &o)
+{
+    SolveRun R;
+    R.o = o;
+    R.mode = o.precision;
+    R.bj = o.precond == AMIE_BLOCK_JACOBI;
+    R.a = B.args(R.mode);
+    if (int rc = team_prepare(B, R, std::vector<char>(B.nprob, 1))) return rc;
+    AMIE_HIP(hipStreamSynchronize(B.stream));   // the copies to the device
+    return AMIE_OK;
+}
+
 // Queues the pass's launch.
 int team_launch(Batch &B, SolveRun &R)
 {
