@@ -5,15 +5,16 @@
 // solve finished (non-blocking event polls), (2) starts the solve of every
 // group whose batch has been built, on its own stream, (3) admits queued
 // requests of one class (element type, right-hand-side count, load kind) as
-// a new group while solve slots and the HBM budget allow, and hands the
-// build of its batch (pattern, layout, assembly on the device) to a host
-// worker thread, and (4) enqueues one more chunk of iterations for every
-// in-flight group.  Builds and the release of finished batches (hipFree
-// synchronises the device) run off the serving thread, so a step never
-// waits for them and in-flight groups keep their chunks coming.  Groups
-// admitted at different times run concurrently on the device, each problem
-// with its own scalars and reductions: a problem's result does not depend
-// on which other problems share its group.
+// a new group while solve slots, the HBM budget and the builds under way
+// allow, and hands the build of its batch (pattern, layout, assembly on the
+// device, team plan) to a host worker thread, and (4) enqueues one more chunk
+// of iterations for every in-flight group that iterates by launches (a team
+// launch runs its pass to the end).  Builds and the release of finished
+// batches (hipFree synchronises the device) run off the serving thread, so a
+// step never waits for them and in-flight groups keep their chunks coming.
+// Groups admitted at different times run concurrently on the device, each
+// problem with its own scalars and reductions: a problem's result does not
+// depend on which other problems share its group.
 // Requests with a persistent key keep their batch (matrix, damage state and
 // solution) resident between requests.  Each such request is one load step
 // in the order of the reference's FeatureTree::stepInternal
@@ -124,12 +125,19 @@ struct Building {
 
 // A group's team launch holds its CUs until the whole pass ends, and team
 // launches of several members run one after the other, while launches of the
-// iteration's phases interleave with the other groups'.  So it has to be
-// expected this much faster (served mix of 2D and 3D cells and damage steps,
-// 419 requests at 200 a second, solves/s with factors 1, 1.5, 2 and never: FP64
-// 52.9, 54.1, 52.5, 54.0, FIX48 95, 93, 82, 79; FP64 at 10 a second, median
-// latency 175, 108, 126, 136 ms).
-constexpr double TEAM_MARGIN = 1.5;
+// iteration's phases interleave with the other groups'.  In FP64, whose teams
+// run longest, one has to be expected this much faster (the served mix at 10
+// requests a second, median latency with factors 1, 1.5, 2 and never: 175, 108,
+// 126, 136 ms; in FIX48 a factor of 1.5 cost a tenth of the throughput at 50).
+constexpr double TEAM_MARGIN_FP64 = 1.5;
+
+// Batches built at a time.  Builds share the context's stream and wait for
+// CUs behind the groups in flight; a request that arrives meanwhile joins the
+// next group instead of a build, a plan and a launch of its own (the served
+// mix at 50 requests a second, FIX48, solves/s with limits 1, 2, 3, 4, 6 and
+// none: 83, 86, 86, 85, 82, 65, at 200 a second 80, 111, 104, 100, 101, 103; FP64
+// at 200 a second 57, 60, 57, 59, 57, 56).
+constexpr int MAX_BUILDING = 3;
 
 template <typename T> static bool ready(std::future<T> &f)
 {
@@ -342,7 +350,7 @@ struct Server {
                 i++;
             }
         }
-        if (!queue.empty() && used_slots < max_slots) {
+        if (!queue.empty() && used_slots < max_slots && (int)building.size() < MAX_BUILDING) {
             const int cls = queue.front().prob.cls();
             const bool pers = queue.front().key != 0;
             std::vector<Request> pick;
@@ -399,7 +407,7 @@ struct Server {
                         return o;
                     }
                     o.rc = batch_create(cx, (int)descs.size(), descs.data(), &o.batch);
-                    if (o.rc == AMIE_OK) o.batch->team_margin = TEAM_MARGIN;
+                    if (o.rc == AMIE_OK) o.batch->team_margin = so.precision == AMIE_FP64 ? TEAM_MARGIN_FP64 : 1.;
                     // the SpMV candidates are timed here too, off the serving thread
                     // (under the load of the groups in flight)
                     const bool tunable = so.precision == AMIE_FP64 || so.precision == AMIE_MIXED ||
