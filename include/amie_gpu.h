@@ -418,14 +418,22 @@ int amie_gpu_batch_set_spmv_kernel(amie_gpu_batch *b, int32_t precision, int32_t
  * leaves it to the library; ALWAYS takes the one launch that keeps the rows
  * on the chip wherever the batch fits it, NEVER one launch per phase.  The
  * results are the same bits.  tiles > 0 sets the tiles (of 256 block rows)
- * a workgroup holds in the one launch, 0 leaves them to the library.  No
+ * a workgroup holds in the one launch, 0 leaves them to the library.
+ *
+ * The workgroups of the one launch wait for each other, so all have to be on
+ * the device at once.  Where that is refused, or a wait sees no progress for
+ * seconds, the pass is finished by launches from the iterate so far, and
+ * AUTO keeps to launches on this batch from then on (amie_gpu_batch_set_team
+ * ends that).  STARVED, for tests, is ALWAYS with too few workgroups for the
+ * first problem that takes several, whose wait gives up at once.  No
  * reference counterpart. */
-enum { AMIE_TEAM_AUTO = 0, AMIE_TEAM_ALWAYS = 1, AMIE_TEAM_NEVER = 2 };
+enum { AMIE_TEAM_AUTO = 0, AMIE_TEAM_ALWAYS = 1, AMIE_TEAM_NEVER = 2, AMIE_TEAM_STARVED = 3 };
 int amie_gpu_batch_set_team(amie_gpu_batch *b, int32_t use, int32_t tiles);
 /* How the latest solve of this batch ran. */
 typedef struct {
     int32_t passes;          /* solve passes */
     int32_t team_passes;     /* of them as one launch */
+    int32_t gave_up;         /* of these, finished by launches */
     int32_t tiles;           /* most tiles a workgroup held in the latest such launch */
     int32_t workgroups;      /* that its problems were cut into */
     int64_t halo_rows;       /* rows of other workgroups that these keep a copy of, summed */

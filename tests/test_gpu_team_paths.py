@@ -105,7 +105,8 @@ def test_team_choice(ctx):
     B = ag.Batch(ctx, probs)
     B.set_team(ag.TEAM_NEVER)
     B.solve(precision=ag.FP64)
-    assert B.team_info() == {"passes": 1, "team_passes": 0, "tiles": 0, "workgroups": 0, "halo_rows": 0}
+    info = B.team_info()
+    assert info["passes"] == 1 and not any(v for k, v in info.items() if k != "passes")
     B.set_team(ag.TEAM_ALWAYS, 2)
     B.solve(precision=ag.FP64)
     info = B.team_info()
@@ -113,7 +114,7 @@ def test_team_choice(ctx):
     assert info == dict(info, passes=1, team_passes=1, tiles=2, workgroups=4)   # 1 681 rows, 7 tiles
     B.solve(precision=ag.MIXED)   # no team kernel for this precision
     assert B.team_info()["team_passes"] == 0
-    for bad in ((3, 0), (-1, 0), (0, -1)):
+    for bad in ((4, 0), (-1, 0), (0, -1)):
         with pytest.raises(ag.AmieError):
             B.set_team(*bad)
     B.close()

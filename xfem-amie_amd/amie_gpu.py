@@ -17,7 +17,7 @@ FP64, MIXED, MIXED64, MIXED_K64, MIXED_SPLIT, MIXED_FIX48 = 0, 1, 2, 3, 4, 5
 DAMAGE_FIBRE, DAMAGE_ISOTROPIC_LINEAR = 0, 1   # event-damage models (amie_event_params.damage_model)
 JACOBI, BLOCK_JACOBI = 0, 1
 REFINE_REPLACE, REFINE_RESTART = 0, 1
-TEAM_AUTO, TEAM_ALWAYS, TEAM_NEVER = 0, 1, 2
+TEAM_AUTO, TEAM_ALWAYS, TEAM_NEVER, TEAM_STARVED = 0, 1, 2, 3
 ASSEMBLE_GATHER, ASSEMBLE_COLOURED = 0, 1
 NPER = {P1: 3, P2: 6, TET4: 4}
 DIM = {P1: 2, P2: 2, TET4: 3}
@@ -73,7 +73,7 @@ class EventStats(ctypes.Structure):
 
 
 class TeamInfo(ctypes.Structure):
-    _fields_ = [("passes", c_i32), ("team_passes", c_i32), ("tiles", c_i32), ("workgroups", c_i32),
+    _fields_ = [("passes", c_i32), ("team_passes", c_i32), ("gave_up", c_i32), ("tiles", c_i32), ("workgroups", c_i32),
                 ("halo_rows", c_i64)]
 
     def as_dict(self):

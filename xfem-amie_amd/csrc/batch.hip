@@ -1124,16 +1124,34 @@ int Batch::start_pass(int mode, const std::vector<char> &subset)
     return AMIE_OK;
 }
 
+// The pass again, by launches, for those of its problems that still run: a
+// team launch was refused or gave up.  Nothing but whole refinements of valid
+// iterates has reached x64.
+int Batch::launch_pass()
+{
+    team_gave_up = true;
+    std::vector<char> left(nprob, 0);
+    for (int p = 0; p < nprob; p++) left[p] = run.was_running[p] && h_prob[p].status == ST_RUNNING;
+    run.info.passes--;
+    return start_pass(run.mode, left);
+}
+
 int Batch::solve_advance()
 {
     SolveRun &R = run;
     if (!R.started || R.finished || R.in_flight) return AMIE_OK;
     hipStream_t s = stream;
     R.nt = 0;
+    if (R.team && !R.persist_launched && team_launch(*this, R)) {
+        // not all of its workgroups fit on the device
+        (void)hipGetLastError();
+        R.info.team_passes++;
+        R.info.gave_up++;
+        if (int rc = launch_pass()) return rc;
+    }
     if (R.pgrid || R.team) {
         // the whole pass in one launch; the status copy follows it
         if (!R.persist_launched && R.team) {
-            if (int rc = team_launch(*this, R)) return rc;
             R.info.team_passes++;
             R.info.tiles = R.team->tpw;
             R.info.workgroups = (int32_t)R.team->h_order.size();
@@ -1184,10 +1202,14 @@ int Batch::solve_poll(bool wait, bool *finished)
         if (!hip_ok(q, "hipEventQuery")) return AMIE_ERR_HIP;
     }
     R.in_flight = false;
-    if ((R.pgrid || R.team) && h_persist_pinned[2]) {
-        if (R.team) team_seq = UINT32_MAX;   // the words' state is unknown: the next pass clears them
-        set_error("%s: a wait gave up (workgroups not all resident?)", R.team ? "team solve" : "persistent solve");
+    if (R.pgrid && h_persist_pinned[2]) {
+        set_error("persistent solve: a wait gave up (workgroups not all resident?)");
         return AMIE_ERR_HIP;
+    }
+    if (R.team && h_persist_pinned[2]) {
+        R.info.gave_up++;
+        std::memcpy(h_prob.data(), h_prob_pinned, nprob * sizeof(ProbDev));
+        return launch_pass();
     }
     if (R.team) team_seq = (uint32_t)h_persist_pinned[3];
     for (int i = 0; i < R.nt; i++) {
@@ -1879,7 +1901,7 @@ int amie_gpu_batch_set_spmv_kernel(amie_gpu_batch *bb, int32_t precision, int32_
 
 int amie_gpu_batch_set_team(amie_gpu_batch *bb, int32_t use, int32_t tiles)
 {
-    if (!bb || !bb->b || use < AMIE_TEAM_AUTO || use > AMIE_TEAM_NEVER || tiles < 0) {
+    if (!bb || !bb->b || use < AMIE_TEAM_AUTO || use > AMIE_TEAM_STARVED || tiles < 0) {
         set_error("bad arguments");
         return AMIE_ERR_ARG;
     }
@@ -1887,6 +1909,7 @@ int amie_gpu_batch_set_team(amie_gpu_batch *bb, int32_t use, int32_t tiles)
     if (B.run.started) { set_error("a solve is in progress"); return AMIE_ERR_BUSY; }
     B.team_use = use;
     B.team_tiles = tiles;
+    B.team_gave_up = false;
     return AMIE_OK;
 }
 

@@ -118,6 +118,7 @@ struct SolveRun {
     const void *team_fn = nullptr;
     size_t team_lds = 0;             // its dynamic LDS
     bool team_single = false;        // every team is one workgroup
+    int team_first = 0;              // the problem whose members are claimed first
     bool persist_launched = false;   // either launch is queued
     amie_team_info info{};
     amie_solve_stats stats{};
@@ -203,6 +204,7 @@ struct Batch {
     uint32_t team_seq = 0;                 // sequence numbers the team CG has used
     bool team_dirty = true;                // p2, p3, p4, y hold launch-path vectors
     int team_use = AMIE_TEAM_AUTO, team_tiles = 0;   // amie_gpu_batch_set_team
+    bool team_gave_up = false;             // a team launch did not get all its workgroups
     double team_margin = 1.;               // how much faster a team launch has to be expected
 
     // captured iteration chunks, keyed by solve variant
@@ -221,6 +223,7 @@ struct Batch {
     int solve(const amie_solve_opts &o, amie_solve_stats *st);
     int solve_begin(const amie_solve_opts &o);
     int start_pass(int mode, const std::vector<char> &subset);
+    int launch_pass();
     int solve_advance();
     int solve_poll(bool wait, bool *finished);
     int solve_end(amie_solve_stats *st);

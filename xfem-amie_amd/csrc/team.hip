@@ -353,7 +353,7 @@ int team_prepare(Batch &B, SolveRun &R, const std::vector<char> &subset)
     R.team = nullptr;
     const int mode = R.mode;
     if ((mode != AMIE_FP64 && mode != AMIE_MIXED_FIX48) || R.o.time_kernels || R.o.persistent > 0 || R.o.use_graph ||
-        B.team_use == AMIE_TEAM_NEVER)
+        B.team_use == AMIE_TEAM_NEVER || B.team_gave_up)
         return AMIE_OK;
     const bool f64 = mode == AMIE_FP64;
     const int b = B.et.b, nr = B.nrhs, w = f64 ? 8 : 4;
@@ -423,6 +423,7 @@ int team_prepare(Batch &B, SolveRun &R, const std::vector<char> &subset)
     R.team_fn = (const void *)fn;
     R.team_lds = dyn;
     R.team_single = single;
+    R.team_first = probs.front();
     return AMIE_OK;
 }
 
@@ -476,7 +477,14 @@ int team_launch(Batch &B, SolveRun &R)
     ta.qh[1] = B.y.as<uint64_t>();
     ta.seq0 = B.team_seq;
     ta.ctl = B.persist.as<uint32_t>();
-    const int grid = std::min(ta.nitems, std::max(1, B.ctx->num_cu));
+    int grid = std::min(ta.nitems, std::max(1, B.ctx->num_cu));
+    if (B.team_use == AMIE_TEAM_STARVED && !R.team_single) {
+        // the largest problem's members come first: one workgroup too few for
+        // them, and the error flag that a wait looks at is set
+        const int p = R.team_first;
+        grid = T.first[p + 1] - T.first[p] - 1;
+        AMIE_HIP(hipMemsetAsync(B.persist.as<char>() + 8, 1, 1, s));
+    }
     AMIE_HIP(hipFuncSetAttribute(R.team_fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)R.team_lds));
     TeamAll all{R.a, ta};
     void *kargs[] = {&all};
@@ -486,6 +494,7 @@ int team_launch(Batch &B, SolveRun &R)
         AMIE_HIP(hipLaunchKernel(R.team_fn, dim3(grid), dim3(TEAM_WG), kargs, R.team_lds, s));
     else
         AMIE_HIP(hipLaunchCooperativeKernel(R.team_fn, dim3(grid), dim3(TEAM_WG), kargs, (unsigned)R.team_lds, s));
+    B.team_seq = UINT32_MAX;   // unknown (the next launch clears the words) until its end is seen
     AMIE_HIP(hipMemcpyAsync(B.h_persist_pinned, B.persist.p, 16, hipMemcpyDeviceToHost, s));
     return AMIE_OK;
 }

@@ -49,7 +49,9 @@
 // members of a problem in a row; a finished workgroup claims the next.  A
 // team waits only for members that resident workgroups will claim, so every
 // wait ends; a wait that sees neither its data nor any team's progress for
-// seconds gives up and ends the launch with an error.
+// seconds gives up and ends the launch.  Its workgroup then publishes nothing
+// and leaves x64 alone, so that x64 only ever holds refinements of valid
+// iterates and the host can finish the pass by launches.
 #pragma once
 #include "device.hpp"
 
@@ -744,8 +746,9 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                 int id;
                 const double tot = wave_sums<1>(&s, lane, id);
                 if (lane == 0) grp[half][g] = tot;
+                if (!ok) s_bad = 1;
                 __syncthreads();
-                if (lane == 0 && g == (NR == 1 ? NGRP - 1 : 0) && v < nv)
+                if (lane == 0 && g == (NR == 1 ? NGRP - 1 : 0) && v < nv && !s_bad)
                     put_sum(total_at(seq, v), (grp[half][0] + grp[half][1]) + (grp[half][2] + grp[half][3]), seq);
                 if (v0 + HALVES * G < nv) __syncthreads();
             }
@@ -1128,7 +1131,8 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                     const double alpha = dn ? 0. : (pq != 0. ? rho / pq : 0.);
                     const double rho1 = mac(alpha * alpha, qmq, mac(-2. * alpha, qz, rho));
                     const double beta = dn ? 0. : (rho != 0. ? rho1 / rho : 0.);
-                    quick = !__any(!dn && (!(pq == pq) || !(rho == rho) || !(qz == qz) || !(qmq == qmq)));
+                    // (nothing more is published after a wait that gave up: its sums are not the others')
+                    quick = !__any(s_bad || (!dn && (!(pq == pq) || !(rho == rho) || !(qz == qz) || !(qmq == qmq))));
                     bool due_now = false;
                     if constexpr (J == 1) {
                         due_now = pending || __any(!dn && rr <= rr_need) || iters + 1 >= due;
@@ -1151,7 +1155,7 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                     if (wave == 0) {
                         int f = 0;
                         if (J == 1 && lane < NR && iters != P.iters && !P.done[lane]) P.rho_pred[lane] = rho_keep;
-                        if (lane == 0) {   // as
+                        if (lane == 0) {
                             P.iters = iters;
                             if (pending) P.ckpt_pending = 1;
                         }
@@ -1241,7 +1245,7 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                 __syncthreads();
                 if (!slot) publish(3 * NR, NVN, xs + 1);
                 else if (tid == 0) P.src_ckpt = 1;
-                if (it == ce - 1 && s_bad) break;   // (a wait that gave up: the quick iterations do not look)
+                if ((it == ce - 1 || H > TEAM_WG) && s_bad) break;   // a halo row's wait gave up
             }
             if (!running || s_bad) break;
             period++;
