@@ -2498,6 +2498,7 @@ int Batch::event_step(const amie_event_params &prm, const amie_solve_opts &o_, a
     amie_solve_opts o = o_;
     o.use_x0 = 1;
     o.use_graph = 0;   // every pass would rebuild the graphs for its active set
+    o.time_kernels = 0;   // the step's stats have no kernel times, and timing them takes the launch path
     const bool small = o.persistent == 0 && small_solvable(B, o);
     if (small) {
         o.precision = AMIE_FP64;
