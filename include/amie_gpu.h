@@ -119,7 +119,8 @@ typedef struct {
                                 tiny system needs a few refinement cycles beyond ndof iterations) */
     int32_t use_x0;          /* 1: start from the current device solution */
     int32_t use_graph;       /* 1: replay hipGraphs of iteration chunks (default 0: plain launches) */
-    int32_t chunk;           /* iterations per chunk between host status checks */
+    int32_t chunk;           /* iterations per chunk between host status checks; a pass in one launch
+                                (see persistent) checks on the device and runs to its end */
     int32_t time_kernels;    /* 1: time every SpMV-kernel launch with HIP events */
     int32_t escalate;        /* AMIE_MIXED: continue stagnating problems in AMIE_FP64 (default 1) */
     int32_t max_grid;        /* > 0: cap on workgroups of the set-up kernels (0: 16 per CU) */
@@ -136,9 +137,12 @@ typedef struct {
                                 the iteration phases separated by device-wide barriers instead of
                                 kernel boundaries; the same results bit for bit.  0 (default):
                                 AMIE_FP64 and AMIE_MIXED_FIX48 run a pass as one launch whose
-                                workgroups keep their rows on the chip, unless time_kernels or
-                                use_graph asks for kernels (again the same results bit for bit);
-                                the other precisions one launch per phase. */
+                                workgroups keep their rows on the chip, where that is expected to
+                                be faster and neither time_kernels nor use_graph asks for kernels
+                                (again the same results bit for bit; amie_gpu_batch_set_team
+                                chooses).  Such a pass ends by convergence, a NaN, stagnation or
+                                maxit; nothing joins or interrupts it before.  Otherwise, and in
+                                the other precisions, one launch per phase. */
 } amie_solve_opts;
 
 typedef struct {
@@ -608,7 +612,12 @@ int amie_gpu_server_release(amie_gpu_server *s, uint64_t persistent_key);
  * left by its last load step; AMIE_ERR_BUSY while it is in flight. */
 int amie_gpu_server_get_damage(amie_gpu_server *s, uint64_t persistent_key, double *d, double *kappa,
                                int64_t nelem);
-/* Advance the solve loop by one chunk (admits, iterates, retires). */
+/* Advance the solve loop: retires finished groups, starts built ones, admits
+ * queued requests (three batches are built at a time) and queues one more
+ * chunk of iterations for every group that iterates by launches; a group
+ * that solves in one launch is done when that is.  Does not wait for the
+ * device, except to read back a finished group's solutions and for a load
+ * step's assembly. */
 int amie_gpu_server_step(amie_gpu_server *s, double now_ms, int32_t *n_active, int32_t *n_queued);
 /* Completed requests since the last poll. */
 int amie_gpu_server_poll(amie_gpu_server *s, amie_request_result *out, int32_t max, int32_t *n);
