@@ -116,7 +116,7 @@ struct SolveRun {
     int pgrid = 0;                   // > 0: this pass runs as one persistent launch of pgrid workgroups
     TeamPlan *team = nullptr;        // this pass runs as one launch of the team CG
     const void *team_fn = nullptr;
-    size_t team_lds = 0;             // its dynamic LDS
+    size_t team_lds = 0, team_lds_most = 0;   // its dynamic LDS, and the most the kernel can have
     bool team_single = false;        // every team is one workgroup
     int team_first = 0;              // the problem whose members are claimed first
     bool persist_launched = false;   // either launch is queued

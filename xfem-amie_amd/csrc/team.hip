@@ -88,6 +88,10 @@ __global__ __launch_bounds__(TEAM_WG) void k_team_halo(SolveArgs a, const TeamMe
 namespace {
 
 constexpr size_t LDS_BYTES = 160 * 1024;
+// The largest dynamic LDS of a kernel is a property of the function, not of a
+// launch: always set to the same, so that batches on other threads (a server
+// builds several at a time) never lower it between here and a launch.
+constexpr size_t HALO_LDS = LDS_BYTES - 8192;   // the bitmap beside k_team_halo's counts
 
 template <typename W> int team_jmax_of(int b, int nr)
 {
@@ -290,7 +294,7 @@ static int team_plan(Batch &B, int tpw, TeamPlan **out)
     }
     T->first[B.nprob] = (int32_t)mem.size();
     const size_t bitmap = (size_t)((rows_max + 31) / 32) * 4;
-    if (bitmap + 8192 > LDS_BYTES || mslice.size() >= INT32_MAX || B.max_width > 65535) T->ok = false;
+    if (bitmap > HALO_LDS || mslice.size() >= INT32_MAX || B.max_width > 65535) T->ok = false;
     if (T->ok) {
         const int nm = (int)mem.size();
         const hipStream_t st = B.stream;
@@ -300,7 +304,7 @@ static int team_plan(Batch &B, int tpw, TeamPlan **out)
             !T->lidx.alloc((size_t)B.nslots * 2) || !T->exported.alloc((size_t)B.nrows_pad) ||
             !T->xb.alloc((size_t)xb * 16) || !T->order.alloc((size_t)nm * 4))
             return no_room();
-        AMIE_HIP(hipFuncSetAttribute((const void *)k_team_halo, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bitmap));
+        AMIE_HIP(hipFuncSetAttribute((const void *)k_team_halo, hipFuncAttributeMaxDynamicSharedMemorySize, (int)HALO_LDS));
         AMIE_HIP(hipMemcpyAsync(T->members.p, mem.data(), nm * sizeof(TeamMember), hipMemcpyHostToDevice, st));
         AMIE_HIP(hipMemcpyAsync(T->mslice.p, mslice.data(), mslice.size() * 4, hipMemcpyHostToDevice, st));
         AMIE_HIP(hipMemcpyAsync(T->mtile.p, mtile.data(), mtile.size() * 4, hipMemcpyHostToDevice, st));
@@ -372,6 +376,7 @@ int team_prepare(Batch &B, SolveRun &R, const std::vector<char> &subset)
     auto fits = [&](TeamFn fn, size_t dyn) -> bool {
         hipFuncAttributes fa{};
         if (hipFuncGetAttributes(&fa, (const void *)fn) != hipSuccess) return false;
+        R.team_lds_most = LDS_BYTES - fa.sharedSizeBytes;
         return fa.sharedSizeBytes + dyn <= LDS_BYTES;
     };
     TeamFn fn = nullptr;
@@ -485,7 +490,7 @@ int team_launch(Batch &B, SolveRun &R)
         grid = T.first[p + 1] - T.first[p] - 1;
         AMIE_HIP(hipMemsetAsync(B.persist.as<char>() + 8, 1, 1, s));
     }
-    AMIE_HIP(hipFuncSetAttribute(R.team_fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)R.team_lds));
+    AMIE_HIP(hipFuncSetAttribute(R.team_fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)R.team_lds_most));
     TeamAll all{R.a, ta};
     void *kargs[] = {&all};
     // members of one team wait for each other: a cooperative launch, which
