@@ -10,10 +10,12 @@ matrix in 48-bit fixed point with FP64 accumulation, FP64 refinement) of all
 volume-averaged stress (effective stiffness) of every RVE.
 
 value = RVE load-case solves per second (1536 per step / step time).
-roofline = the kernel with the larger share of the timed steps, the CG
-update (k_update) or the SpMV (k_spmv), both timed with HIP events on the
-library stream during the timed steps and both reported
-(roofline_update, roofline_spmv).  k_update: the algorithmic bytes of every
+roofline = the dominant kernel of the timed steps: k_cg_team, which runs a
+whole solve pass in one launch (its bytes: the FP32 SpMVs' of the solve).
+Beside it the launch path's two kernels, the CG update (k_update) and the
+SpMV (k_spmv), timed with HIP events during one untimed step by launches
+after the timed ones, which leaves the same solutions (roofline_update,
+roofline_spmv; launch_path_step).  k_update: the algorithmic bytes of every
 launch (27 B per DOF and right-hand side on average: y += alpha p is added
 every fourth iteration, four terms at once) over the kernel time.  k_spmv: the
 algorithmic bytes of the FP32 block SpMV (nnzb (b^2 4 + 4) + 4 (nb + 1) +
@@ -684,22 +686,27 @@ def main():
     ms_per_step = 1e3 * elapsed / args.steps
     solves = len(problems) * problems[0].nrhs
     value = solves * args.steps / elapsed
-    # kernel by kernel (the rooflines): one more step, untimed, on the launch
-    # path, whose SpMV and update are kernels of their own
+    # accuracy sample: six RVEs at the quantiles of n, as the timed steps left
+    # them, against the CPU oracle
+    by_n = np.argsort([p.ndofnodes for p in problems], kind="stable")
+    sample = sorted({int(by_n[int(q * (len(problems) - 1))]) for q in (0., .2, .4, .6, .8, 1.)})
+    x_at = {args.rtol: {k: B.solution(k).copy() for k in sample}}
+    rate_at = {args.rtol: value}
+    team, b8_step = B.team_info(), launches_8d()
+    # kernel by kernel (roofline_spmv, roofline_update): one more step,
+    # untimed, on the launch path, whose SpMV and update are kernels of their
+    # own; it leaves the same solutions
     t0 = time.perf_counter()
     timed, _ = step(headline, time_kernels=1)
-    log(f"launch-path step: {1e3 * (time.perf_counter() - t0):.1f} ms")
+    launch_step = {"ms": 1e3 * (time.perf_counter() - t0), "status": timed["status"],
+                   "solutions_equal_timed": bool(all(np.array_equal(B.solution(k), x_at[args.rtol][k]) for k in sample))}
+    log(f"launch-path step: {launch_step}")
     b8 = launches_8d()
     spmv_ms, spmv_bytes, launches = timed["spmv_kernel_ms"], timed["spmv_bytes"], timed["spmv_launches"]
     upd_ms, upd_bytes, upd_launches = timed["update_kernel_ms"], timed["update_bytes"], timed["update_launches"]
     achieved = b8 / (spmv_ms * 1e-3) / 1e9 if spmv_ms > 0 else 0.0
     achieved_phys = spmv_bytes / (spmv_ms * 1e-3) / 1e9 if spmv_ms > 0 else 0.0
     ok = all(s["status"] == 0 for s in sts)
-    # accuracy sample: six RVEs at the quantiles of n, against the CPU oracle
-    by_n = np.argsort([p.ndofnodes for p in problems], kind="stable")
-    sample = sorted({int(by_n[int(q * (len(problems) - 1))]) for q in (0., .2, .4, .6, .8, 1.)})
-    x_at = {args.rtol: {k: B.solution(k).copy() for k in sample}}
-    rate_at = {args.rtol: value}
 
     def other(precision, name, **kw):
         t1 = time.perf_counter()
@@ -830,7 +837,8 @@ def main():
                                f"assembly + solve + effective stiffness per step",
                    "rves": len(problems), "load_cases": problems[0].nrhs, "dofs": ndof, "blocks": nnzb,
                    "hbm_bytes": hbm_bytes, "converged": ok},
-        "roofline": None,   # the dominant kernel's, set below
+        "roofline": None,   # the dominant kernel's of the timed steps, set below
+        "launch_path_step": launch_step,
         "roofline_spmv": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
                      "bytes": "algorithmic bytes of the FP32 block SpMV per launch: nnzb (b^2 4 + 4) + 4 (nb + 1) + "
@@ -883,8 +891,21 @@ def main():
               "launches": upd_launches, "avg_launch_us": 1e3 * upd_ms / max(1, upd_launches),
               "avg_bytes_per_launch": avg_upd, "kernel_ms": upd_ms, "spmv_kernel_ms": spmv_ms}
     out["roofline_update"] = update
-    # the roofline line is the kernel with the larger share of the timed steps
+    # the roofline line is the dominant kernel of the timed steps: the team CG,
+    # or, where they ran by launches, the kernel with the larger share
     out["roofline"] = dict(update) if upd_ms > spmv_ms else dict(out["roofline_spmv"])
+    if team["team_passes"]:
+        solve_ms = sts[-1]["solve_ms"]
+        out["roofline"] = {
+            "bound": "latency", "achieved": b8_step / (solve_ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": b8_step / (solve_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
+            "traffic": None,
+            "bytes": "algorithmic bytes of the FP32 block SpMVs of the last timed step's solve (as roofline_spmv), over "
+                     "the solve's time, against the HBM peak; the kernel keeps the iteration's vectors on the chip and "
+                     "reads 4 bytes a block (value index, local column), so the memory does not bound it: its "
+                     "wavefronts wait 58 % of their cycles (profiles/team_cg.md)",
+            "kernel": "k_cg_team (a whole solve pass in one launch: product, sums, scalars and update)",
+            "solve_ms": solve_ms, "team": team}
     print(json.dumps(out), flush=True)
 
 
