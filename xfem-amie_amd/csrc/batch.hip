@@ -1124,14 +1124,15 @@ int Batch::start_pass(int mode, const std::vector<char> &subset)
     return AMIE_OK;
 }
 
-// The pass again, by launches, for those of its problems that still run: a
-// team launch was refused or gave up.  Nothing but whole refinements of valid
-// iterates has reached x64.
+// The pass again, by launches, for those of its problems that have not
+// converged: a team launch was refused or gave up (after which a NaN may come
+// from sums that were not all read).  Nothing but refinements of valid
+// iterates has reached x64, and a problem converges by those alone.
 int Batch::launch_pass()
 {
     team_gave_up = true;
     std::vector<char> left(nprob, 0);
-    for (int p = 0; p < nprob; p++) left[p] = run.was_running[p] && h_prob[p].status == ST_RUNNING;
+    for (int p = 0; p < nprob; p++) left[p] = run.was_running[p] && h_prob[p].status != ST_CONVERGED;
     run.info.passes--;
     return start_pass(run.mode, left);
 }

@@ -49,9 +49,11 @@
 // members of a problem in a row; a finished workgroup claims the next.  A
 // team waits only for members that resident workgroups will claim, so every
 // wait ends; a wait that sees neither its data nor any team's progress for
-// seconds gives up and ends the launch.  Its workgroup then publishes nothing
-// and leaves x64 alone, so that x64 only ever holds refinements of valid
-// iterates and the host can finish the pass by launches.
+// seconds gives up and ends the launch.  Its workgroup may publish sums of
+// what it did not get until its period ends, but the error flag is visible
+// before they are, and is looked at before a refinement: x64 only ever holds
+// refinements of valid iterates, a problem converges by their residuals only,
+// and the host finishes the others by launches.
 #pragma once
 #include "device.hpp"
 
@@ -151,6 +153,7 @@ struct TeamWait {
         }
         if (now - since < TEAM_PATIENCE) return true;
         __hip_atomic_store(ctl + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_s_waitcnt(0);   // before anything that follows
         return false;
     }
 };
@@ -746,9 +749,8 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                 int id;
                 const double tot = wave_sums<1>(&s, lane, id);
                 if (lane == 0) grp[half][g] = tot;
-                if (!ok) s_bad = 1;
                 __syncthreads();
-                if (lane == 0 && g == (NR == 1 ? NGRP - 1 : 0) && v < nv && !s_bad)
+                if (lane == 0 && g == (NR == 1 ? NGRP - 1 : 0) && v < nv)
                     put_sum(total_at(seq, v), (grp[half][0] + grp[half][1]) + (grp[half][2] + grp[half][3]), seq);
                 if (v0 + HALVES * G < nv) __syncthreads();
             }
@@ -832,6 +834,13 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
             P.src_ckpt = 1;
         }
         __syncthreads();
+
+        // whether any workgroup of the launch gave up, for all threads after
+        // the next barrier: before a refinement writes x64
+        auto look = [&] {
+            uint32_t *ctl = team_args_of<false>()->t.ctl;
+            if (tid == 0 && __hip_atomic_load(ctl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) s_bad = 1;
+        };
 
         // ---- a refinement: x64 += S y, y = 0 (k_ckpt_x), then r64 =
         // b - K x64, r = S r64, p = M r + beta p (k_ckpt_r).  The residual
@@ -1131,8 +1140,7 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                     const double alpha = dn ? 0. : (pq != 0. ? rho / pq : 0.);
                     const double rho1 = mac(alpha * alpha, qmq, mac(-2. * alpha, qz, rho));
                     const double beta = dn ? 0. : (rho != 0. ? rho1 / rho : 0.);
-                    // (nothing more is published after a wait that gave up: its sums are not the others')
-                    quick = !__any(s_bad || (!dn && (!(pq == pq) || !(rho == rho) || !(qz == qz) || !(qmq == qmq))));
+                    quick = !__any(!dn && (!(pq == pq) || !(rho == rho) || !(qz == qz) || !(qmq == qmq)));
                     bool due_now = false;
                     if constexpr (J == 1) {
                         due_now = pending || __any(!dn && rr <= rr_need) || iters + 1 >= due;
@@ -1242,10 +1250,11 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                         rec_store<W, B, NR>(pl, po);
                         rec_store<W, B, NR>(rl, ro);
                     });
+                if (slot && G > 1) look();
                 __syncthreads();
                 if (!slot) publish(3 * NR, NVN, xs + 1);
                 else if (tid == 0) P.src_ckpt = 1;
-                if ((it == ce - 1 || H > TEAM_WG) && s_bad) break;   // a halo row's wait gave up
+                if (it == ce - 1 && s_bad) break;   // (a wait that gave up: the quick iterations do not look)
             }
             if (!running || s_bad) break;
             period++;
