@@ -11,7 +11,8 @@ volume-averaged stress (effective stiffness) of every RVE.
 
 value = RVE load-case solves per second (1536 per step / step time).
 roofline = the dominant kernel of the timed steps: k_cg_team, which runs a
-whole solve pass in one launch (its bytes: the FP32 SpMVs' of the solve).
+whole solve pass in one launch (its bytes: the stored matrix and local
+columns of every product).
 Beside it the launch path's two kernels, the CG update (k_update) and the
 SpMV (k_spmv), timed with HIP events during one untimed step by launches
 after the timed ones, which leaves the same solutions (roofline_update,
@@ -693,6 +694,7 @@ def main():
     x_at = {args.rtol: {k: B.solution(k).copy() for k in sample}}
     rate_at = {args.rtol: value}
     team, b8_step = B.team_info(), launches_8d()
+    products = sum(shapes[k][1] * (B.problem_info(k)["iterations"] + 1) for k in range(len(problems)))   # blocks
     # kernel by kernel (roofline_spmv, roofline_update): one more step,
     # untimed, on the launch path, whose SpMV and update are kernels of their
     # own; it leaves the same solutions
@@ -895,15 +897,15 @@ def main():
     # or, where they ran by launches, the kernel with the larger share
     out["roofline"] = dict(update) if upd_ms > spmv_ms else dict(out["roofline_spmv"])
     if team["team_passes"]:
-        solve_ms = sts[-1]["solve_ms"]
+        solve_ms, per_block = sts[-1]["solve_ms"], 4 if tf.get("format") == 1 else 26
+        b_team = per_block * products
         out["roofline"] = {
-            "bound": "latency", "achieved": b8_step / (solve_ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "frac": b8_step / (solve_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
-            "traffic": None,
-            "bytes": "algorithmic bytes of the FP32 block SpMVs of the last timed step's solve (as roofline_spmv), over "
-                     "the solve's time, against the HBM peak; the kernel keeps the iteration's vectors on the chip and "
-                     "reads 4 bytes a block (value index, local column), so the memory does not bound it: its "
-                     "wavefronts wait 58 % of their cycles (profiles/team_cg.md)",
+            "bound": "latency", "achieved": b_team / (solve_ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": b_team / (solve_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, "traffic": None,
+            "bytes": f"{per_block} bytes a block (value and local column) of every product of the last timed step's solve, "
+                     "over the solve's time, against the HBM peak.  The iteration's vectors stay on the chip, so the "
+                     "memory does not bound it: the wavefronts wait 58 % of their cycles (profiles/team_cg.md)",
+            "achieved_fp32_yardstick": b8_step / (solve_ms * 1e-3) / 1e9,
             "kernel": "k_cg_team (a whole solve pass in one launch: product, sums, scalars and update)",
             "solve_ms": solve_ms, "team": team}
     print(json.dumps(out), flush=True)
