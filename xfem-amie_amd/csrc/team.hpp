@@ -41,8 +41,10 @@
 // 62 -> 48, P2 400^2 61 -> 42.  What bounds it: on small problems the dependent
 // chain of one iteration (product, transposing sums, one exchange of 1.5 us,
 // scalars, update); on large ones the latency of the matrix stream at 8
-// wavefronts a CU, and the spread of the members' times, which the exchange
-// waits for.
+// wavefronts a CU (P2 400^2 reads 106 MB an iteration at 2.4 TB/s, Tet4 64^3 132
+// at 2.7, a copy runs at 6.3; wavefronts wait 58-66 % of their cycles), the
+// members' halo words, and the spread of the members' times, which the exchange
+// waits for.  Where that makes launches faster they run (team.hip).
 //
 // The workgroups of a launch (at most one per CU, launched cooperatively, so
 // all are resident) claim members in a fixed order from a counter, all
