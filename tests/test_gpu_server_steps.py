@@ -15,8 +15,8 @@ pytestmark = pytest.mark.gpu
 def test_step_starts_a_group_without_waiting(precision):
     """Two cells of 448 and 440 cells a side, in two groups built at the same
     time, to rel. res 1e-12 (some 200 ms each): the second is started while
-    the first is in flight, and no step takes as long as a quarter of the
-    first solve."""
+    the first is in flight, and no step takes as long as half of the first
+    solve (a step that waits takes nearly all of it)."""
     big, small = configs.rve(448, 1, 0.3), configs.rve(440, 2, 0.3)
     ctx = ag.Context(0)
     B = ag.Batch(ctx, [big])
@@ -47,6 +47,6 @@ def test_step_starts_a_group_without_waiting(precision):
     assert list(got.values()) == [0, 0]
     before = [s for k, s in enumerate(steps[:last]) if k not in busy]
     print("alone", alone, "longest step", max(before), flush=True)
-    assert max(before) < 0.25 * alone
+    assert max(before) < 0.5 * alone
     S.close()
     ctx.close()

@@ -87,9 +87,10 @@ struct TeamPlan {
     std::vector<int32_t> nhalo;      // per member: rows of others that it keeps
     std::vector<int32_t> h_order;    // members in the order they are claimed, as on the device
     DevBuf members, order, mslice, mtile, lidx, halo, exported, xb;
+    DevBuf count, loc;               // of the making of it: kept, since freeing them would wait for the device
     size_t bytes() const
     {
-        return members.n + order.n + mslice.n + mtile.n + lidx.n + halo.n + exported.n + xb.n;
+        return members.n + order.n + mslice.n + mtile.n + lidx.n + halo.n + exported.n + xb.n + count.n + loc.n;
     }
 };
 

@@ -298,9 +298,8 @@ static int team_plan(Batch &B, int tpw, TeamPlan **out)
     if (T->ok) {
         const int nm = (int)mem.size();
         const hipStream_t st = B.stream;
-        DevBuf count, dloc;
         if (!T->members.alloc(nm * sizeof(TeamMember)) || !T->mslice.alloc(mslice.size() * 4) ||
-            !T->mtile.alloc(mtile.size() * 4) || !dloc.alloc(loc.size() * 4) || !count.alloc((size_t)nm * 4) ||
+            !T->mtile.alloc(mtile.size() * 4) || !T->loc.alloc(loc.size() * 4) || !T->count.alloc((size_t)nm * 4) ||
             !T->lidx.alloc((size_t)B.nslots * 2) || !T->exported.alloc((size_t)B.nrows_pad) ||
             !T->xb.alloc((size_t)xb * 16) || !T->order.alloc((size_t)nm * 4))
             return no_room();
@@ -308,21 +307,21 @@ static int team_plan(Batch &B, int tpw, TeamPlan **out)
         AMIE_HIP(hipMemcpyAsync(T->members.p, mem.data(), nm * sizeof(TeamMember), hipMemcpyHostToDevice, st));
         AMIE_HIP(hipMemcpyAsync(T->mslice.p, mslice.data(), mslice.size() * 4, hipMemcpyHostToDevice, st));
         AMIE_HIP(hipMemcpyAsync(T->mtile.p, mtile.data(), mtile.size() * 4, hipMemcpyHostToDevice, st));
-        AMIE_HIP(hipMemcpyAsync(dloc.p, loc.data(), loc.size() * 4, hipMemcpyHostToDevice, st));
+        AMIE_HIP(hipMemcpyAsync(T->loc.p, loc.data(), loc.size() * 4, hipMemcpyHostToDevice, st));
         AMIE_HIP(hipMemsetAsync(T->exported.p, 0, T->exported.n, st));
         AMIE_HIP(hipMemsetAsync(T->xb.p, 0, T->xb.n, st));
         AMIE_HIP(hipMemsetAsync(T->lidx.p, 0, T->lidx.n, st));   // the null slots read row 0
         const SolveArgs a = B.args(AMIE_FP64);
         auto halo = [&](int fill) {
             hipLaunchKernelGGL(k_team_halo, dim3(nm), dim3(TEAM_WG), bitmap, st, a, T->members.as<TeamMember>(),
-                               T->mslice.as<int32_t>(), dloc.as<uint32_t>(), B.row_len.as<int32_t>(), fill,
-                               count.as<int32_t>(), T->halo.as<uint32_t>(), T->lidx.as<uint16_t>(),
+                               T->mslice.as<int32_t>(), T->loc.as<uint32_t>(), B.row_len.as<int32_t>(), fill,
+                               T->count.as<int32_t>(), T->halo.as<uint32_t>(), T->lidx.as<uint16_t>(),
                                T->exported.as<uint8_t>());
         };
         halo(0);
         AMIE_HIP(hipGetLastError());
         std::vector<int32_t> h(nm);
-        AMIE_HIP(hipMemcpyAsync(h.data(), count.p, (size_t)nm * 4, hipMemcpyDeviceToHost, st));
+        AMIE_HIP(hipMemcpyAsync(h.data(), T->count.p, (size_t)nm * 4, hipMemcpyDeviceToHost, st));
         AMIE_HIP(hipStreamSynchronize(st));
         int64_t total = 0;
         for (int i = 0; i < nm; i++) {
