@@ -837,13 +837,6 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
         }
         __syncthreads();
 
-        // whether any workgroup of the launch gave up, for all threads after
-        // the next barrier: before a refinement writes x64
-        auto look = [&] {
-            uint32_t *ctl = team_args_of<false>()->t.ctl;
-            if (tid == 0 && __hip_atomic_load(ctl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) s_bad = 1;
-        };
-
         // ---- a refinement: x64 += S y, y = 0 (k_ckpt_x), then r64 =
         // b - K x64, r = S r64, p = M r + beta p (k_ckpt_r).  The residual
         // sums (value 3 NR on) are published for the exchange after it.
@@ -1177,7 +1170,13 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                                            ck);
                         }
                         for (int k = 1; k < NR; k++) f |= __shfl(f, k, WAVE);
-                        if (lane == 0) reduce_finish(P, f, ck);
+                        if (lane == 0) {
+                            reduce_finish(P, f, ck);
+                            // a refinement comes: whether any workgroup gave up
+                            if (G > 1 && it == ce - 1 && P.ckpt_pending &&
+                                __hip_atomic_load(team_args_of<false>()->t.ctl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                                s_bad = 1;
+                        }
                     }
                     __syncthreads();
                     if (s_bad) break;
@@ -1252,7 +1251,6 @@ __global__ __launch_bounds__(TEAM_WG) void k_cg_team(TeamAll all_)
                         rec_store<W, B, NR>(pl, po);
                         rec_store<W, B, NR>(rl, ro);
                     });
-                if (slot && G > 1) look();
                 __syncthreads();
                 if (!slot) publish(3 * NR, NVN, xs + 1);
                 else if (tid == 0) P.src_ckpt = 1;
